@@ -82,8 +82,9 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
         raise ValueError("sinks must be f32 [q_heads]")
     lib = _lib.load()
     pos_dtype = _INDEX[context_q_positions.dtype] if use_context_positions else _lib.AKV_I64
+    window = int(sliding_window_size) if sliding_window_size is not None else -1
     with _on_device(q_extend.device):
-        rc = lib.akv_context_attention(
+        args = (
             q_extend.data_ptr(), q_extend.stride(0), q_extend.stride(1),
             k_extend.data_ptr(), v_extend.data_ptr(), k_extend.stride(0), k_extend.stride(1),
             v_extend.stride(0), v_extend.stride(1),
@@ -93,11 +94,31 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
             qo_indptr.data_ptr(), kv_indptr.data_ptr(), _INDEX[qo_indptr.dtype],
             kv_indices.data_ptr() if kv_indices.numel() else None, _INDEX[kv_indices.dtype],
             _lib.ptr(context_q_positions), _lib.ptr(context_kv_positions), pos_dtype,
-            int(sliding_window_size) if sliding_window_size is not None else -1,
-            _lib.ptr(sinks), float(scale), float(logit_cap), o_extend.data_ptr(),
+            window, _lib.ptr(sinks), float(scale), float(logit_cap), o_extend.data_ptr(),
             _lib.AKV_F32 if o_extend.dtype == torch.float32 else _lib.AKV_BF16,
             o_extend.stride(0), o_extend.stride(1), int(max_len_extend),
-            current_stream_handle(q_extend.device),
         )
+        workspace = _split_workspace(lib, q_extend, n_seg, k_extend.shape[1], window, int(max_len_extend),
+                                     kv_indices.numel())
+        stream = current_stream_handle(q_extend.device)
+        if workspace is None:
+            rc = lib.akv_context_attention(*args, stream)
+        else:
+            rc = lib.akv_context_attention_split(*args, workspace.data_ptr(), workspace.numel(), stream)
     _lib.check(rc, "akv_context_attention")
     return o_extend
+
+
+def _split_workspace(lib, q, n_seg, kv_heads, window, max_query_len, total_prefix):
+    """Workspace of the split launch, or None when the plain one serves the batch.
+
+    From the caching allocator on the current stream, so it is the call's own.
+    """
+    need = lib.akv_context_attention_split_bytes(n_seg, q.shape[1], kv_heads, q.shape[2], window, q.shape[0],
+                                                 max_query_len, total_prefix)
+    if need <= 0:
+        return None
+    try:
+        return torch.empty(need, dtype=torch.uint8, device=q.device)
+    except torch.OutOfMemoryError:
+        return None  # the plain launch needs none

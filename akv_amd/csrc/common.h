@@ -29,6 +29,25 @@ __device__ __forceinline__ int64_t load_index(const void* p, bool is64, int64_t 
               : static_cast<int64_t>(static_cast<const int32_t*>(p)[i]);
 }
 
+// First position in [0, n) whose value is at least `first` (n when none): the
+// 64 lanes probe evenly spaced positions at once, so a long prefix takes three
+// rounds of loads instead of a binary search's fifteen.
+template <typename F>
+__device__ __forceinline__ int32_t first_at_least(F value, int32_t n, int64_t first, int lane) {
+  int32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const int32_t step = (hi - lo + 63) >> 6;
+    const int64_t at = lo + static_cast<int64_t>(lane) * step;
+    const bool below = at < hi && value(static_cast<int32_t>(at < hi ? at : hi - 1)) < first;
+    const int cnt = __builtin_popcountll(__builtin_amdgcn_ballot_w64(below));
+    if (cnt == 0) break;
+    const int64_t next = lo + static_cast<int64_t>(cnt) * step;
+    lo += (cnt - 1) * step + 1;
+    if (next < hi) hi = static_cast<int32_t>(next);
+  }
+  return lo;
+}
+
 __device__ __forceinline__ void store_index(void* p, bool is64, int64_t i, int64_t v) {
   if (is64)
     static_cast<int64_t*>(p)[i] = v;

@@ -57,9 +57,11 @@
 // supplies A[l%16][k(l,i)], B[k(l,i)][l%16] for i < 8 and holds
 // D[4(l/16)+i][l%16]; ds_read_b64_tr_b16 -- within each 16-lane group, lane
 // j receives element j%4 of the 8-byte rows read by lanes j/4 + 4i, i < 4.
+#include <algorithm>
 #include <cmath>
 
 #include "common.h"
+#include "context_plan.h"
 
 namespace akv {
 namespace {
@@ -81,7 +83,15 @@ constexpr int sub_tiles(int d) { return d == 64 ? 4 : 2; }
 // workgroups (half the tile loads per flop, and twice the math per tile to
 // hide each tile's load behind)
 constexpr int kWaves = 8;
-constexpr int rows_per_block(int d) { return kWaves * 16 * sub_tiles(d); }  // (token, head) rows
+// (token, head) rows of a block with `sub` row subtiles per wave
+constexpr int block_rows(int sub) { return kWaves * 16 * sub; }
+constexpr int rows_per_block(int d) { return block_rows(sub_tiles(d)); }
+// Windows up to kNarrowWindow at head_dim 64 take blocks of kNarrowSub subtiles per wave.  A
+// block of few tokens sees few keys outside its rows' windows, and its tiles
+// are short, where a 128-key window's cost is mostly one tile's latency after
+// another; wide windows share each tile over as many rows as full layers do.
+constexpr int kNarrowWindow = 512;
+constexpr int kNarrowSub = 1;
 constexpr int kThreads = 64 * kWaves;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazy = 8.f;  // log2-domain slack before an exact maximum moves
@@ -110,6 +120,10 @@ struct CtxArgs {
   int32_t group, group_shift, tokens_per_block, kv_heads;
   int32_t head_dim;   // head dims in use (<= the kernel's D; the rest are zero)
   float cap, cap_log2;  // logit cap (scores -> cap tanh(score / cap)), cap log2(e)
+  // split launch only
+  int32_t n_segments;
+  int32_t max_shift;    // log2 of the workgroups
+  float* partial;       // kPartialFloats per part, two parts per workgroup
 };
 
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
@@ -182,30 +196,195 @@ __device__ __forceinline__ int32_t rel_pos(int64_t p, int64_t base) {
   return static_cast<int32_t>(r < -kFar ? -kFar : (r > kFar ? kFar : r));
 }
 
+// Workgroups of a split launch: one per CU (a power of two).
+constexpr int kSplitShift = 8;
+constexpr int kSplitGroups = 1 << kSplitShift;
+// The split launch keeps a batch's segments one to a lane.
+constexpr int kMaxSplitSegments = 64;
+
+// One wave's copy of the batch: lane s holds segment s.
+struct BatchPlan {
+  int32_t q0, k0;  // this lane's segment: first query, first prefix index
+  int32_t q, p;    // queries and prefix keys
+  int32_t before;  // cost of the segments before it
+  int32_t total;   // one head's cost
+  uint64_t live;   // segments with queries
+};
+
+template <int D, int KEYS>
+__device__ __forceinline__ SplitShape split_shape(const CtxArgs& a) {
+  return SplitShape{__builtin_ctz(rows_per_block(D)) - a.group_shift, __builtin_ctz(KEYS)};
+}
+
+__device__ __forceinline__ BatchPlan plan_batch(const CtxArgs& a, const SplitShape& sh, int lane) {
+  BatchPlan b;
+  const bool in = lane < a.n_segments;
+  const int s = in ? lane : 0;
+  const int64_t q0 = load_index(a.qo_indptr, a.indptr_i64, s), q1 = load_index(a.qo_indptr, a.indptr_i64, s + 1);
+  const int64_t k0 = load_index(a.kv_indptr, a.indptr_i64, s), k1 = load_index(a.kv_indptr, a.indptr_i64, s + 1);
+  b.q0 = static_cast<int32_t>(q0);
+  b.k0 = static_cast<int32_t>(k0);
+  b.q = in ? static_cast<int32_t>(q1 - q0) : 0;
+  b.p = in && a.kv_indices ? static_cast<int32_t>(k1 - k0) : 0;
+  const int32_t cost = segment_cost(sh, b.q, b.p);
+  int32_t sum = cost;
+#pragma nounroll
+  for (int off = 1; off < a.n_segments; off <<= 1) {
+    const int32_t up = __shfl_up(sum, off);
+    if (lane >= off) sum += up;
+  }
+  b.before = sum - cost;
+  b.total = __builtin_amdgcn_readlane(sum, a.n_segments - 1);
+  b.live = __builtin_amdgcn_ballot_w64(cost > 0);
+  return b;
+}
+
+// Boundary r of this lane (the lanes' searches run side by side).
+__device__ __forceinline__ Place lane_place(const BatchPlan& b, const SplitShape& sh, int32_t heads, int k, int r) {
+  auto get = [&](int i, int32_t* q, int32_t* p, int32_t* before) {
+    *q = __builtin_amdgcn_readlane(b.q, i);
+    *p = __builtin_amdgcn_readlane(b.p, i);
+    *before = __builtin_amdgcn_readlane(b.before, i);
+  };
+  return place_of(sh, get, b.live, b.total, heads, k, r);
+}
+
+__device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ Place uniform(const Place& p) {
+  return Place{uniform(p.head), uniform(p.seg), uniform(p.block), uniform(p.tile)};
+}
+
+__device__ __forceinline__ Place from_lane(const Place& p, int lane) {
+  return Place{__builtin_amdgcn_readlane(p.head, lane), __builtin_amdgcn_readlane(p.seg, lane),
+               __builtin_amdgcn_readlane(p.block, lane), __builtin_amdgcn_readlane(p.tile, lane)};
+}
+
+// Stores a row's normalised output, from its O (4 dims of each of TILES 16-dim
+// tiles from dt0 on), weight sum l and maximum m (-inf: the row has seen no
+// key), with the sink.
+template <int D, bool GEN, int TILES>
+__device__ __forceinline__ void store_row(const CtxArgs& a, int g, int r, int32_t t0, int32_t qlen, int64_t qo0,
+                                          int quad, int dt0, const f32x4 (&o)[TILES], float l, float m_run) {
+  const int G = a.group;
+  const int hl = r & ((1 << a.group_shift) - 1);
+  float scale = 1.f;
+  if (a.sinks) {
+    const float sink = a.sinks[g * G + (GEN && hl >= G ? G - 1 : hl)] * kLog2e;
+    const float m_f = fmaxf(m_run, sink);
+    scale = m_run == -INFINITY ? 0.f : exp2f(m_run - m_f);
+    l = l * scale + exp2f(sink - m_f);
+  }
+  const float inv = l > 0.f ? scale / l : 0.f;
+  const int32_t row_token = r >> a.group_shift, row_head = g * G + hl;
+  if (t0 + row_token >= qlen || (GEN && hl >= G)) return;
+  const int64_t at = (qo0 + t0 + row_token) * a.o_st + static_cast<int64_t>(row_head) * a.o_sh + 16 * dt0 + 4 * quad;
+#pragma unroll
+  for (int dt = 0; dt < TILES; ++dt) {
+    if (GEN && 16 * (dt0 + dt) + 4 * quad >= a.head_dim) continue;
+    const f32x4 v = o[dt] * inv;
+    if (a.out_f32) {
+      *reinterpret_cast<f32x4*>(static_cast<float*>(a.out) + at + 16 * dt) = v;
+    } else {
+      bf16x4 ob;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) ob[i] = static_cast<__bf16>(v[i]);
+      *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(a.out) + at + 16 * dt) = ob;
+    }
+  }
+}
+
+// A partial result: O of every (16-dim tile, row subtile) as the lanes hold it
+// (whole 1 KiB stores), then each row's maximum and weight sum.
+constexpr int kPartialO = 32768;  // rows_per_block(D) * D floats, either head_dim
+template <int D>
+constexpr int64_t partial_floats() { return kPartialO + 2 * rows_per_block(D); }
+
+// Where a stretch starts (tile -1: no such stretch), with its segment's first
+// query and query count.  The workspace ends with one for every workgroup.
+struct __attribute__((aligned(16))) Cut {
+  Place at;
+  int32_t q0, q, pad[2];
+};
+
+template <int D>
+__device__ __forceinline__ Cut* split_cuts(const CtxArgs& a) {
+  return reinterpret_cast<Cut*>(a.partial + 2 * kSplitGroups * partial_floats<D>());
+}
+
+// A segment's first query and prefix index, its queries and prefix keys.
+struct Segment {
+  int64_t q0, k0;
+  int32_t q, p;
+};
+
+template <int D, int KEYS, int SUB>
+struct Lds {
+  TileLds<D, KEYS>& tile0;
+  TileLds<D, KEYS>& tile1;
+  int32_t (&rel_rows)[block_rows(SUB)];
+  int32_t& restart_flag;
+  float2* merge;  // 4 x 16 SUB, split launch only
+};
+
+struct SplitState {
+  Place cur, first, end;
+  uint64_t live;  // segments with queries
+  int32_t rank;
+  int32_t last;  // the part left for last is the one being done
+};
+
+// The next block, segment or head after s.cur in its stretch, then the part
+// left for last; false when the stretch is done.  qlen: s.cur's segment.
+__device__ __forceinline__ bool next_piece(const CtxArgs& a, SplitState& s, int32_t qlen) {
+  if (s.last) return false;
+  bool done = same_block(s.cur, s.end);
+  if (!done) {
+    s.cur.tile = 0;
+    if ((s.cur.block + 1) * a.tokens_per_block < qlen) {
+      ++s.cur.block;
+    } else {
+      s.cur.block = 0;
+      const uint64_t later = s.cur.seg < 63 ? s.live >> (s.cur.seg + 1) << (s.cur.seg + 1) : 0;
+      if (!later) ++s.cur.head;
+      s.cur.seg = __builtin_ctzll(later ? later : s.live);
+    }
+    done = s.cur.head >= a.kv_heads || (same_block(s.cur, s.end) && s.end.tile == 0);
+  }
+  if (!done) return true;
+  if (s.first.tile == 0 || same_block(s.first, s.end)) return false;
+  s.cur = s.first;
+  s.last = 1;
+  return true;
+}
+
 // KEYS keys per tile: 128 for full layers at head_dim 64 (half the tile
 // barriers, staging and commits per key), 64 for windowed layers (less of a
 // tile outside the window) and at head_dim 128 (measured faster than 128 there)
 // GEN: the general instance -- logit caps, heads narrower than D (the dims
 // past head_dim zero in the tiles), groups padded to a power of two; the
 // plain instance takes none of these checks.
-template <int D, int KEYS, typename IdxT, typename PosT, bool POS, bool GEN>
-__global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const CtxArgs a) {
-  constexpr int kSub = sub_tiles(D);
+//
+// One block of queries of a segment for KV head `g`, over its key tiles
+// [it_first, it_stop) (it_stop < 0: to the end; a plain launch's are all of
+// them).  All the workgroup's threads call it.  `part`: where a split launch
+// keeps a part of a block's result.
+template <int D, int KEYS, int SUB, typename IdxT, typename PosT, bool POS, bool GEN, bool SPLIT>
+__device__ __forceinline__ void attend(const CtxArgs& a, const Lds<D, KEYS, SUB>& lds, const Segment& sg, int g,
+                                       int32_t block, int it_first, int it_stop, float* part) {
+  const int it_begin = SPLIT ? it_first : 0;
+  constexpr int kSub = SUB;
   constexpr int kKeys = KEYS;
   constexpr int kChunks = D / 8;               // 16 B chunks per key row
   constexpr int kKSteps = D / 32;              // MFMA k-steps over head dims
   constexpr int kDTiles = D / 16;              // O^T row tiles
-  __shared__ __attribute__((aligned(16))) TileLds<D, KEYS> tile0, tile1;
-
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // uniform: LDS block bases in SGPRs
   const int col = lane & 15;
   const int quad = lane >> 4;
-  const int seg = blockIdx.z;
-  const bool i64 = a.indptr_i64;
-  const int64_t qo0 = load_index(a.qo_indptr, i64, seg);
-  const int32_t qlen = static_cast<int32_t>(load_index(a.qo_indptr, i64, seg + 1) - qo0);
+  const int64_t qo0 = sg.q0;
+  const int32_t qlen = sg.q;
   const int G = a.group;                         // q heads per KV head
   const int gmask = (1 << a.group_shift) - 1;    // rows per token: G padded to a power of two
   const int T = a.tokens_per_block;
@@ -214,18 +393,9 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
   // the score's log2-domain multiplier: with a cap the scores are capped
   // (and scaled) before the softmax, which then takes them as they are
   const float mult = cap ? 1.f : a.scale_log2;
-  // KV head fastest: workgroup id mod 8 picks the XCD, so with 8 KV heads
-  // every XCD streams one head's K/V through its own L2.  Token blocks run
-  // last-first: the last blocks see the most causal keys, and starting them
-  // first shortens the tail of the launch.
-  const int g = static_cast<int>(blockIdx.x % static_cast<unsigned>(a.kv_heads));
-  const int32_t t0 = static_cast<int32_t>(gridDim.x / static_cast<unsigned>(a.kv_heads) - 1 -
-                                          blockIdx.x / static_cast<unsigned>(a.kv_heads)) * T;
-  if (t0 >= qlen) return;
-  const int64_t kv0 = load_index(a.kv_indptr, i64, seg);
-  // without prefix indices there is no prefix, whatever kv_indptr says
-  const int32_t plen =
-      a.kv_indices ? static_cast<int32_t>(load_index(a.kv_indptr, i64, seg + 1) - kv0) : 0;
+  const int32_t t0 = block * T;
+  const int64_t kv0 = sg.k0;
+  const int32_t plen = sg.p;
   // segment-local views
   const PosT* qpos = static_cast<const PosT*>(a.q_pos) + qo0;
   const PosT* kpos = static_cast<const PosT*>(a.kv_pos) + kv0;
@@ -248,59 +418,24 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
     if constexpr (POS) return static_cast<int64_t>(kpos[j]);
     return static_cast<int64_t>(j);
   };
+  const int window = SPLIT ? -1 : a.window;  // a split launch has none
   const int64_t qbase = qpos_of(t0);
   const int32_t e_hi = qlen < t0 + T ? qlen : t0 + T;  // extend keys [e_lo, e_hi)
   const int32_t last_rel = rel_pos(qpos_of(e_hi - 1), qbase);
 
   // keys below qbase - window are outside every row's window
   int32_t p_lo = 0, e_lo = 0;
-  if (a.window >= 0) {
-    const int64_t first = qbase - a.window;
-    int32_t lo = 0, hi = plen;
-    while (lo < hi) {
-      const int32_t mid = (lo + hi) >> 1;
-      if (kpos_of(mid) < first) lo = mid + 1; else hi = mid;
-    }
-    p_lo = lo;
-    lo = 0;
-    hi = t0;
-    while (lo < hi) {
-      const int32_t mid = (lo + hi) >> 1;
-      if (qpos_of(mid) < first) lo = mid + 1; else hi = mid;
-    }
-    e_lo = lo;
+  if (window >= 0) {
+    const int64_t first = qbase - window;
+    p_lo = first_at_least(kpos_of, plen, first, lane);
+    e_lo = first_at_least(qpos_of, t0, first, lane);
   }
   const int n_pref = (plen - p_lo + kKeys - 1) / kKeys;
   const int n_tiles = n_pref + (e_hi - e_lo + kKeys - 1) / kKeys;
+  const int it_end = !SPLIT || it_stop < 0 ? n_tiles : it_stop;
   auto tile_base = [&](int it) -> int32_t {
     return it < n_pref ? p_lo + it * kKeys : e_lo + (it - n_pref) * kKeys;
   };
-
-  // this lane's rows: row subtile s covers rows wave * 16 kSub + 16s + col,
-  // row r = (token r >> group_shift, q head g G + r % G); the rows'
-  // positions relative to qbase wait in LDS for the masked tiles
-  __shared__ int32_t rel_rows[rows_per_block(D)];
-  auto row_of = [&](int s) { return wave * (16 * kSub) + 16 * s + col; };
-  bf16x8 qop[kSub][kKSteps];
-#pragma unroll
-  for (int s = 0; s < kSub; ++s) {
-    const int r = row_of(s);
-    const int tl = r >> a.group_shift;
-    const int hl = r & gmask;
-    const int head = g * G + hl;
-    const bool tok = t0 + tl < qlen;
-    // a padding row (hl >= G) keeps Q = 0 and is never stored
-    const bool ok = tok && (!GEN || hl < G);
-    if (quad == 0) rel_rows[r] = tok ? rel_pos(qpos_of(t0 + tl), qbase) : last_rel;
-#pragma unroll
-    for (int ks = 0; ks < kKSteps; ++ks) {
-      u32x4 w = {0u, 0u, 0u, 0u};
-      // head dims past hd are zero
-      if (ok && (!GEN || 8 * (4 * ks + quad) < hd))
-        w = load16(a.q + (qo0 + t0 + tl) * a.q_st + static_cast<int64_t>(head) * a.q_sh + 32 * ks + 8 * quad);
-      qop[s][ks] = __builtin_bit_cast(bf16x8, w);
-    }
-  }
 
   // tile staging straight into LDS (global_load_lds_dwordx4: lane l of a
   // wave instruction fills bytes 16 l of a 1 KiB block).  Block b of a tile
@@ -360,7 +495,7 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
       }
     }
     // key positions matter only to a window (causal masking is by index)
-    if (a.window >= 0 && tid < kKeys) {
+    if (window >= 0 && tid < kKeys) {
       // loaded now, converted at commit: no wait on the tile's row loads here
       const int32_t j = base + tid;
       const int32_t end = ext ? e_hi : plen;
@@ -373,9 +508,53 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
   // the barrier that follows publishes the whole tile
   auto commit = [&](TileLds<D, KEYS>& t) {
     // (without a window every key's position reads 0, which the mask admits)
-    if (tid < kKeys) t.pos[tid] = a.window < 0 ? 0 : (pvalid ? rel_pos(preg, qbase) : kFar);
+    if (tid < kKeys) t.pos[tid] = window < 0 ? 0 : (pvalid ? rel_pos(preg, qbase) : kFar);
     __builtin_amdgcn_s_waitcnt(0);
   };
+
+  // the first tile's slots are on their way while Q loads
+  if (it_begin < n_pref) fetch_slots(it_begin);
+
+  // this lane's rows: row subtile s covers rows group * 16 kSub + 16s + col,
+  // row r = (token r >> group_shift, q head g G + r % G); the rows'
+  // positions relative to qbase wait in LDS for the masked tiles.  A split
+  // launch's short block has 1, 2 or 4 groups of rows; its waves then share
+  // the 32-key quarters of each tile (wave w takes row group w % groups and
+  // quarters w / groups, w / groups + sharers, ...) and merge at the end.
+  int groups = kWaves, sharers = 1;
+  if constexpr (SPLIT) {
+    const int32_t rows = (qlen - t0 < T ? qlen - t0 : T) << a.group_shift;
+    while (groups > 1 && rows <= (groups >> 1) * (16 * kSub)) {
+      groups >>= 1;
+      sharers <<= 1;
+    }
+  }
+  const int row_group = SPLIT ? wave & (groups - 1) : wave;
+  const int share = SPLIT ? wave / groups : 0;
+  auto row_of = [&](int s) { return row_group * (16 * kSub) + 16 * s + col; };
+  bf16x8 qop[kSub][kKSteps];
+#pragma unroll
+  for (int s = 0; s < kSub; ++s) {
+    const int r = row_of(s);
+    const int tl = r >> a.group_shift;
+    const int hl = r & gmask;
+    const int head = g * G + hl;
+    const bool tok = t0 + tl < qlen;
+    // rows past the segment are never stored: a split launch, whose pieces are
+    // short, repeats its last query there (no branch around the loads), the
+    // plain one keeps Q = 0; a padding row (hl >= G) keeps Q = 0
+    const int32_t tr = SPLIT && !tok ? qlen - 1 : t0 + tl;
+    const bool ok = (SPLIT || tok) && (!GEN || hl < G);
+    if (quad == 0) lds.rel_rows[r] = tok ? rel_pos(qpos_of(t0 + tl), qbase) : last_rel;
+#pragma unroll
+    for (int ks = 0; ks < kKSteps; ++ks) {
+      u32x4 w = {0u, 0u, 0u, 0u};
+      // head dims past hd are zero
+      if (ok && (!GEN || 8 * (4 * ks + quad) < hd))
+        w = load16(a.q + (qo0 + tr) * a.q_st + static_cast<int64_t>(head) * a.q_sh + 32 * ks + 8 * quad);
+      qop[s][ks] = __builtin_bit_cast(bf16x8, w);
+    }
+  }
 
   f32x4 oacc[kDTiles][kSub];
   // per row: the negated running maximum -m (log2 domain; 0 while the row
@@ -398,8 +577,7 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
   bool unset = true;
   // after a restart every tile takes the exact maxima (uniform)
   bool exact_all = false;
-  __shared__ int32_t restart_flag;
-  if (tid == 0) restart_flag = 0;
+  if (tid == 0) lds.restart_flag = 0;
   const bf16x8 kOnes = {__bf16(1.f), __bf16(1.f), __bf16(1.f), __bf16(1.f),
                         __bf16(1.f), __bf16(1.f), __bf16(1.f), __bf16(1.f)};
 
@@ -409,20 +587,22 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
     // land before any wave's direct loads into tile 0: barrier first.
     constexpr int kWords = KEYS * D / 8;  // 16 B chunks per array
     for (int i = tid; i < 4 * kWords; i += kThreads) {
-      __bf16* arr = i < kWords ? &tile0.k[0][0] : i < 2 * kWords ? &tile0.v[0][0]
-                  : i < 3 * kWords ? &tile1.k[0][0] : &tile1.v[0][0];
+      __bf16* arr = i < kWords ? &lds.tile0.k[0][0] : i < 2 * kWords ? &lds.tile0.v[0][0]
+                  : i < 3 * kWords ? &lds.tile1.k[0][0] : &lds.tile1.v[0][0];
       reinterpret_cast<u32x4*>(arr)[i % kWords] = u32x4{0u, 0u, 0u, 0u};
     }
     __syncthreads();
   }
-  if (n_pref > 0) fetch_slots(0);
-  stage(0, tile0);
-  if (1 < n_pref) fetch_slots(1);
-  commit(tile0);
-  __syncthreads();
+  auto open = [&]() {
+    stage(it_begin, lds.tile0);
+    if (it_begin + 1 < n_pref) fetch_slots(it_begin + 1);
+    commit(lds.tile0);
+    __syncthreads();
+  };
+  open();
   // tile it from cur while tile it + 1 streams into nxt
   auto step = [&](int it, TileLds<D, KEYS>& cur, TileLds<D, KEYS>& nxt) {
-    if (it + 1 < n_tiles) {
+    if (it + 1 < it_end) {
       stage(it + 1, nxt);
       if (it + 2 < n_pref) fetch_slots(it + 2);
     }
@@ -433,7 +613,7 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
     // masking is needed for a partial tile, keys past the block's first
     // query (causal), or keys older than the last query's window
     const bool masked = count < kKeys || (ext && base + kKeys - 1 > t0) ||
-                        (a.window >= 0 && __builtin_amdgcn_readfirstlane(cur.pos[0]) < last_rel - a.window);
+                        (window >= 0 && __builtin_amdgcn_readfirstlane(cur.pos[0]) < last_rel - window);
     const bool exact = unset || exact_all;
 
     // The tile in quarters of 32 keys (kk), each complete before the next:
@@ -488,7 +668,7 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
           const int r = row_of(s);
           const int32_t climit = ext ? t0 + (r >> a.group_shift) - base : kKeys;
           const int32_t last = climit < count - 1 ? climit : count - 1;
-          const int32_t thr = a.window >= 0 ? rel_rows[r] - a.window : -kFar - 1;
+          const int32_t thr = window >= 0 ? lds.rel_rows[r] - window : -kFar - 1;
 #pragma unroll
           for (int j = 0; j < 2; ++j) {
             const int k0 = 16 * (2 * kk + j) + 4 * quad;
@@ -555,7 +735,10 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
           oacc[dt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[s], oacc[dt][s], 0, 0, 0);
       }
     };
-    if constexpr (kKeys == 64) {
+    if constexpr (SPLIT) {
+#pragma nounroll
+      for (int kk = share; kk < kKeys / 32; kk += sharers) half(kk);
+    } else if constexpr (kKeys == 64) {
       half(0);
       half(1);
     } else {
@@ -577,7 +760,7 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
       huge |= lacc[s][0] > kHuge;
     }
     if (__builtin_amdgcn_ballot_w64(big)) {
-      if (!exact && __builtin_amdgcn_ballot_w64(huge)) restart_flag = 1;
+      if (!exact && __builtin_amdgcn_ballot_w64(huge)) lds.restart_flag = 1;
       // sum -> [1/2, 1): O and the sum by 2^-e, the maximum up by e
 #pragma unroll
       for (int s = 0; s < kSub; ++s) {
@@ -597,110 +780,369 @@ __global__ void __launch_bounds__(kThreads, 2) context_attention_kernel(const Ct
       for (int s = 0; s < kSub; ++s) none |= lacc[s][0] == 0.f;
       unset = __builtin_amdgcn_ballot_w64(none) != 0;
     }
-    if (it + 1 < n_tiles) commit(nxt);
+    if (it + 1 < it_end) commit(nxt);
     __syncthreads();
   };
   // a restart (decided before the tile's barrier, read after it by every
   // wave) starts the keys again from tile 0 with exact maxima; no load is in
   // flight after a barrier and neither buffer is still being read
   auto restart_flag_set = [&]() -> bool {
-    return !exact_all && __builtin_amdgcn_readfirstlane(*static_cast<volatile int32_t*>(&restart_flag));
+    return !exact_all && __builtin_amdgcn_readfirstlane(*static_cast<volatile int32_t*>(&lds.restart_flag));
   };
   auto restarted = [&]() -> bool {
     if (!restart_flag_set()) return false;
     exact_all = true;
     unset = true;
     clear_rows();
-    if (n_pref > 0) fetch_slots(0);
-    stage(0, tile0);
-    if (1 < n_pref) fetch_slots(1);
-    commit(tile0);
-    __syncthreads();
+    if (it_begin < n_pref) fetch_slots(it_begin);
+    open();
     return true;
   };
-  for (int it = 0; it < n_tiles; it += 2) {
-    step(it, tile0, tile1);
+  for (int it = it_begin; it < it_end; it += 2) {
+    step(it, lds.tile0, lds.tile1);
     // a restart after the first half skips the second
-    if (it + 1 < n_tiles && !restart_flag_set()) step(it + 1, tile1, tile0);
-    if (restarted()) it = -2;
+    if (it + 1 < it_end && !restart_flag_set()) step(it + 1, lds.tile1, lds.tile0);
+    if (restarted()) it = it_begin - 2;
   }
 
-  // normalise with the sink; store
+  if constexpr (SPLIT) {
+    // merge the sharers of each row group through the tiles' LDS (free after
+    // the last tile's barrier), the upper half into the lower half
+    for (int half_sharers = sharers >> 1; half_sharers > 0; half_sharers >>= 1) {
+      const bool gives = share >= half_sharers && share < 2 * half_sharers, takes = share < half_sharers;
+      const int region = (gives ? share - half_sharers : share) * groups + row_group;  // below 4
+      // 16 KB of O, two regions to a tile buffer, and the rows' (m, l)
+      f32x4* ro = reinterpret_cast<f32x4*>(region < 2 ? &lds.tile0.k[0][0] : &lds.tile1.k[0][0]) + (region & 1) * 1024;
+      float2* rm = lds.merge + region * (16 * kSub);
+      if (gives) {
 #pragma unroll
-  for (int s = 0; s < kSub; ++s) {
-    float l = lacc[s][0];
-    float scale = 1.f;
-    const int hl = row_of(s) & gmask;
-    if (a.sinks) {
-      const float m_run = l != 0.f ? -neg_m[s] : -INFINITY;
-      const float sink = a.sinks[g * G + (GEN && hl >= G ? G - 1 : hl)] * kLog2e;
-      const float m_f = fmaxf(m_run, sink);
-      scale = m_run == -INFINITY ? 0.f : exp2f(m_run - m_f);
-      l = l * scale + exp2f(sink - m_f);
+        for (int s = 0; s < kSub; ++s) {
+#pragma unroll
+          for (int dt = 0; dt < kDTiles; ++dt) ro[(dt * kSub + s) * 64 + lane] = oacc[dt][s];
+          if (quad == 0) rm[16 * s + col] = float2{lacc[s][0] != 0.f ? -neg_m[s] : -INFINITY, lacc[s][0]};
+        }
+      }
+      __syncthreads();
+      if (takes) {
+#pragma unroll
+        for (int s = 0; s < kSub; ++s) {
+          const float2 ml = rm[16 * s + col];
+          const float m0 = lacc[s][0] != 0.f ? -neg_m[s] : -INFINITY;
+          const float mn = fmaxf(m0, ml.x);
+          const float w0 = m0 == -INFINITY ? 0.f : exp2f(m0 - mn), w1 = ml.x == -INFINITY ? 0.f : exp2f(ml.x - mn);
+          lacc[s][0] = lacc[s][0] * w0 + ml.y * w1;
+          neg_m[s] = mn == -INFINITY ? 0.f : -mn;
+#pragma unroll
+          for (int dt = 0; dt < kDTiles; ++dt)
+            oacc[dt][s] = oacc[dt][s] * w0 + ro[(dt * kSub + s) * 64 + lane] * w1;
+        }
+      }
+      __syncthreads();
     }
-    const float inv = l > 0.f ? scale / l : 0.f;
-    const int32_t row_token = row_of(s) >> a.group_shift, row_head = g * G + hl;
-    if (t0 + row_token >= qlen || (GEN && hl >= G)) continue;
-    const int64_t at =
-        (qo0 + t0 + row_token) * a.o_st + static_cast<int64_t>(row_head) * a.o_sh + 4 * quad;
+    if (share != 0) return;
+  }
+
+  // a block whose keys are all here is normalised with the sink and stored; a
+  // part of one goes to the workspace
+  if (!SPLIT || (it_begin == 0 && it_end == n_tiles)) {
 #pragma unroll
-    for (int dt = 0; dt < kDTiles; ++dt) {
-      if (GEN && 16 * dt + 4 * quad >= hd) continue;
-      const f32x4 o = oacc[dt][s] * inv;
-      if (a.out_f32) {
-        *reinterpret_cast<f32x4*>(static_cast<float*>(a.out) + at + 16 * dt) = o;
-      } else {
-        bf16x4 ob;
+    for (int s = 0; s < kSub; ++s) {
+      f32x4 o[kDTiles];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) ob[i] = static_cast<__bf16>(o[i]);
-        *reinterpret_cast<bf16x4*>(static_cast<__bf16*>(a.out) + at + 16 * dt) = ob;
+      for (int dt = 0; dt < kDTiles; ++dt) o[dt] = oacc[dt][s];
+      const float l = lacc[s][0];
+      store_row<D, GEN, kDTiles>(a, g, row_of(s), t0, qlen, qo0, quad, 0, o, l, l != 0.f ? -neg_m[s] : -INFINITY);
+    }
+  } else {
+#pragma unroll
+    for (int s = 0; s < kSub; ++s) {
+#pragma unroll
+      for (int dt = 0; dt < kDTiles; ++dt)
+        reinterpret_cast<f32x4*>(part)[(dt * kSub + s) * kThreads + tid] = oacc[dt][s];
+      const float l = lacc[s][0];
+      if (quad == 0) {
+        part[kPartialO + 2 * row_of(s)] = l != 0.f ? -neg_m[s] : -INFINITY;
+        part[kPartialO + 2 * row_of(s) + 1] = l;
       }
     }
   }
 }
 
-template <int D, int KEYS, typename IdxT, bool GEN>
-void launch_pos(int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
-  // pos: 0 none, 1 int32, 2 int64
-  if (pos == 2)
-    hipLaunchKernelGGL((context_attention_kernel<D, KEYS, IdxT, int64_t, true, GEN>), grid, dim3(kThreads), 0, st, a);
-  else if (pos == 1)
-    hipLaunchKernelGGL((context_attention_kernel<D, KEYS, IdxT, int32_t, true, GEN>), grid, dim3(kThreads), 0, st, a);
-  else
-    hipLaunchKernelGGL((context_attention_kernel<D, KEYS, IdxT, int64_t, false, GEN>), grid, dim3(kThreads), 0, st,
-                       a);
+template <int D, int KEYS, int SUB, typename IdxT, typename PosT, bool POS, bool GEN>
+__global__ void __launch_bounds__(kThreads, SUB == 1 ? 4 : 2) context_attention_kernel(const CtxArgs a) {
+  __shared__ __attribute__((aligned(16))) TileLds<D, KEYS> tile0, tile1;
+  __shared__ int32_t rel_rows[block_rows(SUB)];
+  __shared__ int32_t restart_flag;
+  const Lds<D, KEYS, SUB> lds{tile0, tile1, rel_rows, restart_flag, nullptr};
+  // KV head fastest: workgroup id mod 8 picks the XCD, so with 8 KV heads
+  // every XCD streams one head's K/V through its own L2.  Token blocks run
+  // last-first: the last blocks see the most causal keys, and starting them
+  // first shortens the tail of the launch.
+  const int g = static_cast<int>(blockIdx.x % static_cast<unsigned>(a.kv_heads));
+  const int32_t block = static_cast<int32_t>(gridDim.x / static_cast<unsigned>(a.kv_heads) - 1 -
+                                             blockIdx.x / static_cast<unsigned>(a.kv_heads));
+  const int seg = blockIdx.z;
+  const bool i64 = a.indptr_i64;
+  Segment sg;
+  sg.q0 = load_index(a.qo_indptr, i64, seg);
+  sg.q = static_cast<int32_t>(load_index(a.qo_indptr, i64, seg + 1) - sg.q0);
+  sg.k0 = load_index(a.kv_indptr, i64, seg);
+  // without prefix indices there is no prefix, whatever kv_indptr says
+  sg.p = a.kv_indices ? static_cast<int32_t>(load_index(a.kv_indptr, i64, seg + 1) - sg.k0) : 0;
+  if (block * a.tokens_per_block >= sg.q) return;
+  attend<D, KEYS, SUB, IdxT, PosT, POS, GEN, false>(a, lds, sg, g, block, 0, -1, nullptr);
 }
 
-template <int D, int KEYS, typename IdxT>
-void launch_cap(int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
+// The split launch: one workgroup per CU, each with an equal stretch of the
+// batch's cost line (context_plan.h).  It is for batches whose plain grid
+// leaves CUs idle: 200 new tokens over 19441 keys are 32 plain workgroups and
+// took 560 us for the GPT-OSS layer, 95 us here with the merge (the matrix
+// cores' share is 52 us; the rest is the cuts, a block's first tile, the parts'
+// 28 MB each way and the second launch); six ragged Llama-3 segments (48-624
+// queries over 4-14k keys) took 594 us, 461 us here.
+//
+// A stretch that starts inside a block leaves that block's part for last: the
+// workgroups of an XCD then all begin at their blocks' first keys and walk
+// the keys of a segment together.  What the loop carries waits in LDS and the
+// arguments are read again for each piece, so the tile loop keeps the scalar
+// registers it has in the plain kernel (held in registers, some 80 of them
+// spilled to vector lanes inside the tile loop, which cost it 15-25%).
+typedef __attribute__((address_space(4))) const CtxArgs kernel_args;
+
+template <int D, int KEYS, typename IdxT, bool GEN>
+__global__ void __launch_bounds__(kThreads, 2) context_split_kernel(const CtxArgs args) {
+  __shared__ __attribute__((aligned(16))) TileLds<D, KEYS> tile0, tile1;
+  __shared__ int32_t rel_rows[rows_per_block(D)];
+  __shared__ int32_t restart_flag;
+  __shared__ float2 merge[4 * 16 * sub_tiles(D)];
+  __shared__ SplitState state;
+  __shared__ int4 segments[kMaxSplitSegments];  // first query and prefix index, queries, prefix keys
+  const Lds<D, KEYS, sub_tiles(D)> lds{tile0, tile1, rel_rows, restart_flag, merge};
+  {
+    const SplitShape shape = split_shape<D, KEYS>(args);
+    const int lane = threadIdx.x & 63;
+    const BatchPlan plan = plan_batch(args, shape, lane);
+    const int k = parts_shift(shape, plan.total, args.kv_heads, args.max_shift);
+    const int id = static_cast<int>(blockIdx.x);
+    if (plan.total == 0 || (id >> k)) {
+      if (threadIdx.x == 0) split_cuts<D>(args)[id].at = Place{0, 0, 0, -1};
+      return;
+    }
+    // workgroup id mod 8 picks the XCD: each XCD gets an eighth of the line
+    SplitState s;
+    s.rank = k >= 3 ? ((id & 7) << (k - 3)) + (id >> 3) : id;
+    s.live = plan.live;
+    const Place ends = lane_place(plan, shape, args.kv_heads, k, s.rank + (lane & 1));
+    s.first = from_lane(ends, 0);
+    s.end = from_lane(ends, 1);
+    s.cur = s.first;
+    s.last = 0;
+    const int32_t qlen = __builtin_amdgcn_readlane(plan.q, s.first.seg);
+    if (threadIdx.x == 0)
+      split_cuts<D>(args)[s.rank] = Cut{s.first, __builtin_amdgcn_readlane(plan.q0, s.first.seg), qlen, {0, 0}};
+    if (same_block(s.first, s.end) ? s.first.tile == s.end.tile
+                                   : s.first.tile > 0 && !next_piece(args, s, qlen))
+      return;
+    if (threadIdx.x == 0) state = s;
+    if (threadIdx.x < kMaxSplitSegments) segments[threadIdx.x] = int4{plan.q0, plan.k0, plan.q, plan.p};
+    __syncthreads();
+  }
+  kernel_args* kp = (kernel_args*)__builtin_amdgcn_kernarg_segment_ptr();
+  for (;;) {
+    asm volatile("" : "+s"(kp));
+    const CtxArgs& a = *(const CtxArgs*)kp;
+    {
+      const Place at = uniform(state.cur), end = uniform(state.end);
+      const int rank = uniform(state.rank);
+      // part 2 rank: the stretch's first block, entered past its first tile;
+      // part 2 rank + 1: its last, left before its last tile
+      float* part = a.partial + (2 * rank + (at.tile > 0 ? 0 : 1)) * partial_floats<D>();
+      const int4 v = segments[at.seg];
+      const Segment sg{uniform(v.x), uniform(v.y), uniform(v.z), uniform(v.w)};
+      attend<D, KEYS, sub_tiles(D), IdxT, int64_t, false, GEN, true>(a, lds, sg, at.head, at.block, at.tile,
+                                                                     same_block(at, end) ? end.tile : -1, part);
+    }
+    SplitState s = state;
+    s.cur = uniform(s.cur);
+    s.first = uniform(s.first);
+    s.end = uniform(s.end);
+    s.live = (static_cast<uint64_t>(static_cast<uint32_t>(uniform(static_cast<int32_t>(s.live >> 32)))) << 32) |
+             static_cast<uint32_t>(uniform(static_cast<int32_t>(s.live)));
+    s.last = uniform(s.last);
+    if (!next_piece(a, s, uniform(segments[s.cur.seg].z))) return;
+    __syncthreads();
+    if (threadIdx.x == 0) state = s;
+    __syncthreads();
+  }
+}
+
+// Merges the parts of each block that a boundary between two stretches cuts.
+// Workgroup = (64 / 32 rows of one wave of the main kernel, boundary); the
+// block's first boundary does the work.  A wave takes one row subtile and two
+// 16-dim tiles, every lane the same rows and dims as in the main kernel, so
+// the parts are read in whole 1 KiB accesses, eight parts at a time: the cost
+// is round trips (the cuts, then the parts), not bandwidth.
+constexpr int kCombineDims = 2;  // 16-dim tiles of a wave
+template <int D, bool GEN>
+__global__ void __launch_bounds__(512) context_combine_kernel(const CtxArgs a) {
+  constexpr int kSub = sub_tiles(D);
+  constexpr int kAhead = 8;  // parts whose loads are in flight together
+  static_assert(64 * kSub * (D / 16 / kCombineDims) == 512, "one wave per row subtile and pair of dim tiles");
+  const int lane = threadIdx.x & 63;
+  const int w = uniform(threadIdx.x >> 6);
+  const int s = w % kSub, dt0 = w / kSub * kCombineDims;
+  const int wave = blockIdx.x;
+  const int r0 = blockIdx.y + 1;
+  // lane i: boundary r0 - 1 + i
+  const Cut* cuts = split_cuts<D>(a);
+  auto load_cut = [&](int r) {
+    Cut c = cuts[r < kSplitGroups ? r : 0];
+    if (r >= kSplitGroups) c.at.tile = -1;
+    return c;
+  };
+  Cut mine = load_cut(r0 - 1 + lane);
+  const Place at = from_lane(mine.at, 1), prev = from_lane(mine.at, 0);
+  // nothing, or a boundary between two blocks, or not the block's first
+  if (at.tile <= 0 || (prev.tile > 0 && same_block(prev, at))) return;
+  const int64_t qo0 = __builtin_amdgcn_readlane(mine.q0, 1);
+  const int32_t qlen = __builtin_amdgcn_readlane(mine.q, 1);
+  const int32_t t0 = at.block * a.tokens_per_block;
+  if (t0 + ((wave * 16 * kSub) >> a.group_shift) >= qlen) return;  // no rows here (nor a part with them)
+  const int row = wave * (16 * kSub) + 16 * s + (lane & 15);
+  f32x4 o[kCombineDims];
+#pragma unroll
+  for (int dt = 0; dt < kCombineDims; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  // the block's parts: its first tiles, up to boundary r0, by the workgroup
+  // before it, then one part from each of its boundaries, unless the next
+  // boundary lies on the same tile
+  int base = r0 - 1, first = 2 * r0 - 1;
+  bool more = true;
+  while (more) {
+    // lane i: boundary base + i and the one after it (lane 63's: not known)
+    const int32_t here = base + lane >= r0 && same_block(mine.at, at) ? mine.at.tile : -1;
+    const int32_t next = __shfl_down(here, 1);
+    more = __builtin_amdgcn_readlane(here, 63) > 0;
+    uint64_t parts = __builtin_amdgcn_ballot_w64(here > 0 && lane < 63 && here != next);
+    while (parts || first >= 0) {
+      f32x4 op[kAhead][kCombineDims];
+      float2 ml[kAhead];
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        int slot = 2 * r0 - 1;  // past the last part: the first one again, with no weight
+        bool has = true;
+        if (first >= 0) {
+          first = -1;
+        } else if (parts) {
+          slot = 2 * (base + __builtin_ctzll(parts));
+          parts &= parts - 1;
+        } else {
+          has = false;
+        }
+        const float* part = a.partial + slot * partial_floats<D>();
+        ml[u] = *reinterpret_cast<const float2*>(part + kPartialO + 2 * row);
+        if (!has) ml[u].x = -INFINITY;
+#pragma unroll
+        for (int dt = 0; dt < kCombineDims; ++dt)
+          op[u][dt] = reinterpret_cast<const f32x4*>(part)[((dt0 + dt) * kSub + s) * kThreads + wave * 64 + lane];
+      }
+      float mn = m;
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) mn = fmaxf(mn, ml[u].x);
+      const float wo = m == -INFINITY ? 0.f : exp2f(m - mn);
+      l *= wo;
+#pragma unroll
+      for (int dt = 0; dt < kCombineDims; ++dt) o[dt] *= wo;
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        // a row without a key in the part (or no part at all) adds nothing
+        const bool none = ml[u].x == -INFINITY;
+        const float wu = none ? 0.f : exp2f(ml[u].x - mn);
+        l += none ? 0.f : ml[u].y * wu;
+#pragma unroll
+        for (int dt = 0; dt < kCombineDims; ++dt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[dt][i] += none ? 0.f : op[u][dt][i] * wu;
+      }
+      m = mn;
+    }
+    base += 63;
+    if (more) mine = load_cut(base + lane);
+  }
+  store_row<D, GEN, kCombineDims>(a, at.head, row, t0, qlen, qo0, lane >> 4, dt0, o, l, m);
+}
+
+// SUB 0: the split launch
+template <int D, int KEYS, int SUB, typename IdxT, bool GEN>
+void launch_pos(int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
+  // pos: 0 none, 1 int32, 2 int64; only a window looks at positions, and
+  // neither a split launch nor one of 128-key tiles has one
+  if constexpr (SUB == 0) {
+    hipLaunchKernelGGL((context_split_kernel<D, KEYS, IdxT, GEN>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((context_combine_kernel<D, GEN>), dim3(kWaves, grid.x - 1), dim3(512), 0, st, a);
+  } else {
+    if (KEYS == 128 || pos == 0)
+      hipLaunchKernelGGL((context_attention_kernel<D, KEYS, SUB, IdxT, int64_t, false, GEN>), grid, dim3(kThreads), 0,
+                         st, a);
+    if constexpr (KEYS != 128) {
+      if (pos == 2)
+        hipLaunchKernelGGL((context_attention_kernel<D, KEYS, SUB, IdxT, int64_t, true, GEN>), grid, dim3(kThreads), 0,
+                           st, a);
+      else if (pos == 1)
+        hipLaunchKernelGGL((context_attention_kernel<D, KEYS, SUB, IdxT, int32_t, true, GEN>), grid, dim3(kThreads), 0,
+                           st, a);
+    }
+  }
+}
+
+template <int D, int KEYS, int SUB, typename IdxT>
+void launch_gen(int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
   // the general instance for caps, narrower heads and padded groups
   if (a.cap > 0.f || a.head_dim != D || a.group != (1 << a.group_shift))
-    launch_pos<D, KEYS, IdxT, true>(pos, grid, st, a);
+    launch_pos<D, KEYS, SUB, IdxT, true>(pos, grid, st, a);
   else
-    launch_pos<D, KEYS, IdxT, false>(pos, grid, st, a);
+    launch_pos<D, KEYS, SUB, IdxT, false>(pos, grid, st, a);
 }
 
-template <int D, int KEYS>
+template <int D, int KEYS, int SUB>
 void launch_idx(bool idx64, int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
   if (idx64)
-    launch_cap<D, KEYS, int64_t>(pos, grid, st, a);
+    launch_gen<D, KEYS, SUB, int64_t>(pos, grid, st, a);
   else
-    launch_cap<D, KEYS, int32_t>(pos, grid, st, a);
+    launch_gen<D, KEYS, SUB, int32_t>(pos, grid, st, a);
 }
 
-void launch_typed(int head_dim, bool idx64, int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
-  if (head_dim > 64)
-    launch_idx<128, 64>(idx64, pos, grid, st, a);
+void launch_typed(bool split, bool idx64, int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
+  const bool wide = a.head_dim > 64;
+  if (split)
+    wide ? launch_idx<128, 64, 0>(idx64, pos, grid, st, a) : launch_idx<64, 128, 0>(idx64, pos, grid, st, a);
+  else if (wide)
+    launch_idx<128, 64, sub_tiles(128)>(idx64, pos, grid, st, a);
+  else if (a.window >= 0 && a.window <= kNarrowWindow)
+    launch_idx<64, 64, kNarrowSub>(idx64, pos, grid, st, a);
   else if (a.window >= 0)
-    launch_idx<64, 64>(idx64, pos, grid, st, a);
+    launch_idx<64, 64, sub_tiles(64)>(idx64, pos, grid, st, a);
   else
-    launch_idx<64, 128>(idx64, pos, grid, st, a);
+    launch_idx<64, 128, sub_tiles(64)>(idx64, pos, grid, st, a);
+}
+
+int group_shift_of(int32_t group) {
+  int s = 0;
+  while ((1 << s) < group) ++s;  // rows per token: the group padded to 2^s
+  return s;
+}
+
+int64_t split_bytes(int32_t head_dim) {
+  return kSplitGroups * (8 * (head_dim > 64 ? partial_floats<128>() : partial_floats<64>()) + sizeof(Cut));
 }
 
 }  // namespace
 }  // namespace akv
 
-extern "C" int akv_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_ext,
+namespace akv {
+namespace {
+
+int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_ext,
                                      const void* v_ext, int64_t k_ext_stride_t, int64_t k_ext_stride_h,
                                      int64_t v_ext_stride_t, int64_t v_ext_stride_h, const void* k_buffer,
                                      const void* v_buffer, int64_t k_stride_slot, int64_t k_stride_head,
@@ -711,8 +1153,7 @@ extern "C" int akv_context_attention(const void* q, int64_t q_stride_t, int64_t 
                                      int32_t positions_dtype, int32_t sliding_window, const float* sinks,
                                      float scale, float logit_cap, void* out, int32_t out_dtype,
                                      int64_t out_stride_t, int64_t out_stride_h, int64_t max_query_len,
-                                     void* stream) {
-  using namespace akv;
+                                     void* workspace, int64_t workspace_bytes, void* stream) {
   if (n_segments < 0 || max_query_len < 0) return fail(AKV_EINVAL, "akv_context_attention: negative size");
   if (n_segments == 0 || max_query_len == 0) return AKV_OK;
   // heads of up to 128 dims in 16-byte chunks: the kernel's 64- or 128-dim
@@ -787,19 +1228,108 @@ extern "C" int akv_context_attention(const void* q, int64_t q_stride_t, int64_t 
   a.scale_log2 = scale * kLog2e;
   a.out_f32 = out_dtype == AKV_F32;
   a.group = q_heads / kv_heads;
-  while ((1 << a.group_shift) < a.group) ++a.group_shift;  // rows per token: the group padded to 2^shift
+  a.group_shift = group_shift_of(a.group);
   const int tile_dim = head_dim > 64 ? 128 : 64;
-  a.tokens_per_block = rows_per_block(tile_dim) >> a.group_shift;
+  const int sub = tile_dim == 64 && a.window >= 0 && a.window <= kNarrowWindow ? kNarrowSub : sub_tiles(tile_dim);
+  a.tokens_per_block = block_rows(sub) >> a.group_shift;
   a.head_dim = head_dim;
   a.cap = logit_cap;
   a.cap_log2 = logit_cap * kLog2e;
   const int64_t blocks = (max_query_len + a.tokens_per_block - 1) / a.tokens_per_block;
   if (blocks * kv_heads > 0x7fffffffLL) return fail(AKV_EINVAL, "akv_context_attention: queries too long");
   a.kv_heads = kv_heads;
-  const dim3 grid(static_cast<unsigned>(blocks * kv_heads), 1u, static_cast<unsigned>(n_segments));
+  const bool split = workspace != nullptr;
+  if (split && (a.window >= 0 || n_segments > kMaxSplitSegments || workspace_bytes < split_bytes(head_dim) ||
+                (reinterpret_cast<uintptr_t>(workspace) & 15) != 0))
+    return fail(AKV_EINVAL, "akv_context_attention_split: needs no window, at most %d segments and %lld aligned bytes",
+                kMaxSplitSegments, static_cast<long long>(split_bytes(head_dim)));
+  a.n_segments = n_segments;
+  a.max_shift = kSplitShift;
+  a.partial = static_cast<float*>(workspace);
+  const dim3 grid = split ? dim3(kSplitGroups)
+                          : dim3(static_cast<unsigned>(blocks * kv_heads), 1u, static_cast<unsigned>(n_segments));
   hipStream_t st = as_stream(stream);
   const bool idx64 = indices_dtype == AKV_I64;
-  const int pos = q_positions == nullptr ? 0 : (positions_dtype == AKV_I64 ? 2 : 1);
-  launch_typed(head_dim, idx64, pos, grid, st, a);
+  const int pos = q_positions == nullptr || a.window < 0 ? 0 : (positions_dtype == AKV_I64 ? 2 : 1);
+  launch_typed(split, idx64, pos, grid, st, a);
   return check_launch("akv_context_attention");
+}
+
+}  // namespace
+}  // namespace akv
+
+extern "C" int akv_context_attention(
+    const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_ext,
+    const void* v_ext, int64_t k_ext_stride_t, int64_t k_ext_stride_h, int64_t v_ext_stride_t, int64_t v_ext_stride_h,
+    const void* k_buffer, const void* v_buffer, int64_t k_stride_slot, int64_t k_stride_head, int64_t v_stride_slot,
+    int64_t v_stride_head, int32_t n_segments, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+    const void* qo_indptr, const void* kv_indptr, int32_t indptr_dtype, const void* kv_indices, int32_t indices_dtype,
+    const void* q_positions, const void* kv_positions, int32_t positions_dtype, int32_t sliding_window,
+    const float* sinks, float scale, float logit_cap, void* out, int32_t out_dtype, int64_t out_stride_t,
+    int64_t out_stride_h, int64_t max_query_len,
+    void* stream) {
+  return akv::run_context_attention(
+      q, q_stride_t, q_stride_h, k_ext, v_ext, k_ext_stride_t, k_ext_stride_h, v_ext_stride_t, v_ext_stride_h, k_buffer,
+      v_buffer, k_stride_slot, k_stride_head, v_stride_slot, v_stride_head, n_segments, q_heads, kv_heads, head_dim,
+      qo_indptr, kv_indptr, indptr_dtype, kv_indices, indices_dtype, q_positions, kv_positions, positions_dtype,
+      sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len,
+      nullptr, 0, stream);
+}
+
+extern "C" int akv_context_attention_split(
+    const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_ext,
+    const void* v_ext, int64_t k_ext_stride_t, int64_t k_ext_stride_h, int64_t v_ext_stride_t, int64_t v_ext_stride_h,
+    const void* k_buffer, const void* v_buffer, int64_t k_stride_slot, int64_t k_stride_head, int64_t v_stride_slot,
+    int64_t v_stride_head, int32_t n_segments, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+    const void* qo_indptr, const void* kv_indptr, int32_t indptr_dtype, const void* kv_indices, int32_t indices_dtype,
+    const void* q_positions, const void* kv_positions, int32_t positions_dtype, int32_t sliding_window,
+    const float* sinks, float scale, float logit_cap, void* out, int32_t out_dtype, int64_t out_stride_t,
+    int64_t out_stride_h, int64_t max_query_len,
+    void* workspace, int64_t workspace_bytes, void* stream) {
+  return akv::run_context_attention(
+      q, q_stride_t, q_stride_h, k_ext, v_ext, k_ext_stride_t, k_ext_stride_h, v_ext_stride_t, v_ext_stride_h, k_buffer,
+      v_buffer, k_stride_slot, k_stride_head, v_stride_slot, v_stride_head, n_segments, q_heads, kv_heads, head_dim,
+      qo_indptr, kv_indptr, indptr_dtype, kv_indices, indices_dtype, q_positions, kv_positions, positions_dtype,
+      sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len,
+      workspace, workspace_bytes, stream);
+}
+
+// Which launch: both times estimated in 64-key tiles of a full block (2.0 us,
+// at either head_dim), from what the host knows.  The plain grid's workgroups
+// run in ceil(groups / CUs) rounds of the longest block (or, of many unequal
+// ones, one round more than they fill), after ~12 us; the
+// split launch shares all tiles out evenly at ~6% more a tile, plus ~10 us for
+// each block a workgroup enters (queries, first tile, result) and ~18 us of
+// its own (the cuts, the second launch).  Measured plain against split, us,
+// GPT-OSS (64 q / 8 KV heads x 64) | Llama-3 (32 / 8 x 128), new tokens over
+// prefix keys: 16 / 1000: 45 / 25 | 39 / 25; 200 / 400: 38 / 42 | 30 / 32;
+// 200 / 1000: 52 / 40 | 46 / 37; 800 / 300: 53 / 56 | 45 / 45; 800 / 5000:
+// 183 / 112 | 185 / 101; 1500 / 5000: 207 / 188 | 207 / 176; 2040 / 19000
+// (one full round): 726 / 780 | 650 / 669; 3000 / 300: 128 / 154 | 109 / 127;
+// 3000 / 5000: 397 / 369 | 388 / 342; 4096 / 19441 (two full rounds): 1310 /
+// 1423 | 1326 / 1381; 6 x 682 / 300: 101 / 113 | 79 / 94; 6 x 682 / 5000: 501
+// / 433 | 502 / 411.
+extern "C" int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t q_heads, int32_t kv_heads,
+                                                     int32_t head_dim, int32_t sliding_window, int64_t total_queries,
+                                                     int64_t max_query_len, int64_t total_prefix) {
+  using namespace akv;
+  if (n_segments <= 0 || n_segments > kMaxSplitSegments || sliding_window > 0 || kv_heads <= 0 || q_heads < kv_heads ||
+      q_heads / kv_heads > 128 || head_dim <= 0 || head_dim > 128 || total_queries <= 0 || max_query_len <= 0)
+    return 0;
+  const int64_t tokens = rows_per_block(head_dim > 64 ? 128 : 64) >> group_shift_of(q_heads / kv_heads);
+  const SplitShape shape{__builtin_ctz(static_cast<uint32_t>(tokens)), head_dim > 64 ? 6 : 7};
+  if (total_prefix < 0 || total_queries > (1 << 30) || total_prefix > (1 << 30) ||
+      cost_bound(shape, n_segments, total_queries, total_prefix) > (1 << 30))
+    return 0;
+  const int64_t queries = n_segments == 1 && max_query_len < total_queries ? max_query_len : total_queries;
+  // one segment's blocks are known; of several, each leaves half a block empty
+  const int64_t blocks = n_segments == 1 ? (queries + tokens - 1) / tokens : queries / tokens + (n_segments + 1) / 2;
+  const int64_t groups = blocks * kv_heads, rounds = (groups + kSplitGroups - 1) / kSplitGroups;
+  const int64_t prefix = total_prefix / n_segments, own = queries / n_segments / 2;
+  const int64_t longest = (n_segments == 1 ? prefix : prefix + prefix / 2) + own;
+  const double share = static_cast<double>(groups) / kSplitGroups, tiles = (prefix + own) / 64.;
+  const double plain = 6. + std::min(rounds * (longest / 64.), (share + 1.) * tiles);
+  const double split = 1.06 * share * tiles + 5. * (share + 1.) + 9.;
+  if (plain <= split) return 0;
+  return split_bytes(head_dim);
 }

@@ -419,6 +419,43 @@ int akv_context_attention(const void* q, int64_t q_stride_t,
                           void* stream);
 
 /*
+ * The same attention with the keys of each block of queries shared out over
+ * one workgroup per CU: for batches without a sliding window whose blocks of
+ * queries would leave CUs idle.  Partial results of blocks whose keys were
+ * cut go to the workspace and a second launch merges them.
+ * akv_context_attention_split_bytes returns the workspace's size for a batch
+ * (total_queries and total_prefix: host bounds of the batch's sums), or 0
+ * when the plain call is the better one.  The workspace holds nothing between
+ * calls; calls that overlap need one each.  At most 64 segments, 16-byte
+ * aligned workspace.
+ */
+int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t q_heads,
+                                          int32_t kv_heads, int32_t head_dim,
+                                          int32_t sliding_window,
+                                          int64_t total_queries,
+                                          int64_t max_query_len,
+                                          int64_t total_prefix);
+int akv_context_attention_split(const void* q, int64_t q_stride_t,
+                          int64_t q_stride_h, const void* k_ext,
+                          const void* v_ext, int64_t k_ext_stride_t,
+                          int64_t k_ext_stride_h, int64_t v_ext_stride_t,
+                          int64_t v_ext_stride_h, const void* k_buffer,
+                          const void* v_buffer, int64_t k_stride_slot,
+                          int64_t k_stride_head, int64_t v_stride_slot,
+                          int64_t v_stride_head, int32_t n_segments,
+                          int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+                          const void* qo_indptr, const void* kv_indptr,
+                          int32_t indptr_dtype, const void* kv_indices,
+                          int32_t indices_dtype, const void* q_positions,
+                          const void* kv_positions, int32_t positions_dtype,
+                          int32_t sliding_window, const float* sinks,
+                          float scale, float logit_cap, void* out,
+                          int32_t out_dtype, int64_t out_stride_t,
+                          int64_t out_stride_h, int64_t max_query_len,
+                          void* workspace, int64_t workspace_bytes,
+                          void* stream);
+
+/*
  * Host (CPU) occurrence window of one forward: the (raw token, position)
  * versions its attention reads and the order in which they are first
  * needed.  Inputs are the compiled layout's int32 vectors (birth positions

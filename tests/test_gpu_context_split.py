@@ -1,0 +1,92 @@
+"""The split prefill launch (keys of a block shared out over workgroups, then
+merged) against the float64 oracle, at the shapes where its cuts can go wrong:
+one block over many workgroups, cuts between blocks, segments and heads,
+segments without queries or prefix, padded groups and narrow heads, partial
+last blocks, and parts whose maxima lie far apart."""
+
+import numpy as np
+import pytest
+import torch
+
+from akv_amd import _lib
+from test_gpu_context_attention import TOL, _case, _run
+
+pytestmark = pytest.mark.gpu
+
+
+def _split(hq, hkv, d, q_lens, p_lens):
+    return _lib.load().akv_context_attention_split_bytes(len(q_lens), hq, hkv, d, -1, sum(q_lens), max(q_lens),
+                                                         sum(p_lens)) > 0
+
+
+CASES = [
+    # d, hq, hkv, queries, prefixes, cap
+    (64, 8, 1, [3], [5000], 0.0),  # one short block over every workgroup it can feed
+    (64, 64, 8, [200], [2500], 0.0),  # full blocks and a short last one
+    (64, 16, 2, [1, 0, 300, 33], [4000, 10, 0, 1500], 0.0),  # no queries / no prefix
+    (64, 32, 4, [64, 128, 65], [1024, 896, 1025], 0.0),  # blocks and tiles exactly full, and one past
+    (128, 32, 8, [33, 257, 64], [1500, 700, 64], 0.0),
+    (128, 4, 1, [1], [3000], 0.0),
+    (64, 3, 3, [700], [1100], 0.0),  # group 1: 512-token blocks
+    (128, 28, 4, [40, 9], [1300, 2000], 0.0),  # padded group
+    (96, 24, 8, [50], [1800], 20.0),  # padded group, narrow head, cap
+    (32, 8, 1, [17, 90], [2100, 5], 0.0),
+]
+
+
+@pytest.mark.parametrize("d,hq,hkv,q_lens,p_lens,cap", CASES)
+@pytest.mark.parametrize("with_sinks,out_dtype", [(False, torch.float32), (True, torch.bfloat16)])
+def test_split_matches_oracle(device, d, hq, hkv, q_lens, p_lens, cap, with_sinks, out_dtype):
+    assert _split(hq, hkv, d, q_lens, p_lens)
+    c = _case(device, hq, hkv, d, q_lens, p_lens, seed=d + hq + len(q_lens), slots=sum(p_lens) + 8)
+    sinks = (torch.randn(hq, generator=torch.Generator().manual_seed(5)) * 2).to(device) if with_sinks else None
+    print(f"split d={d} hq={hq} hkv={hkv} q={q_lens} p={p_lens} cap={cap} sinks={with_sinks}", flush=True)
+    got, want = _run(device, c, window=-1, positions=False, sinks=sinks, out_dtype=out_dtype, scale=d ** -0.5,
+                     logit_cap=cap)
+    assert np.abs(got - want).max() <= TOL
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(64, 8, 1), (128, 8, 2)])
+@pytest.mark.parametrize("step", [-300.0, -60.0, 30.0, 70.0, 300.0])
+def test_split_parts_far_apart(device, d, hq, hkv, step):
+    """Scores that step by ``step`` (log2 domain) every 500 prefix keys, so
+    the parts' maxima differ by up to thousands: the merge keeps the largest
+    part and drops what underflows beside it."""
+    q_lens, p_lens = [20], [3000]
+    assert _split(hq, hkv, d, q_lens, p_lens)
+    c = _case(device, hq, hkv, d, q_lens, p_lens, seed=int(step) + 400, slots=4000)
+    rng = np.random.default_rng(3)
+    c["idx"] = (rng.permutation(3999)[:3000] + 1).astype(np.int32)
+    c["q"][..., 0] = 8.0
+    unit = d ** -0.5 * 1.4426950408889634 * 8.0
+    for j in range(0, 3000, 500):
+        c["kp"][torch.from_numpy(c["idx"][j:j + 500]).long(), :, 0] = step * (j // 500) / unit
+    c["dev"]["q"], c["dev"]["kp"] = c["q"].to(device), c["kp"].to(device)
+    print(f"split parts far apart d={d} step={step}", flush=True)
+    got, want = _run(device, c, window=-1, positions=False, sinks=None, out_dtype=torch.float32, scale=d ** -0.5)
+    assert np.isfinite(got).all()
+    assert np.abs(got - want).max() <= TOL
+
+
+@pytest.mark.parametrize("positions", [True, False])
+@pytest.mark.parametrize("window", [1, 511, 512, 513, 700])
+def test_windows_at_the_block_size_rule(device, window, positions):
+    """Windows up to 512 take blocks of few tokens, wider ones full blocks."""
+    c = _case(device, 16, 2, 64, [300, 17], [900, 40], seed=window)
+    got, want = _run(device, c, window=window, positions=positions, sinks=None, out_dtype=torch.float32, scale=0.125)
+    assert np.abs(got - want).max() <= TOL
+
+
+def test_split_rejects_a_window_and_a_short_workspace():
+    lib = _lib.load()
+    assert lib.akv_context_attention_split_bytes(1, 64, 8, 64, 128, 200, 200, 20000) == 0
+    assert lib.akv_context_attention_split_bytes(65, 64, 8, 64, -1, 6500, 100, 20000) == 0
+    assert lib.akv_context_attention_split_bytes(1, 64, 8, 64, -1, 4096, 4096, 20000) == 0
+    fn = lib.akv_context_attention_split
+    args = [None if t is _lib.c_void_p else 0 for t in fn.argtypes]
+    fake = 1 << 20
+    for i, v in {0: fake, 3: fake, 4: fake, 15: 1, 16: 8, 17: 1, 18: 64, 19: fake, 20: fake, 29: 0.125, 31: fake,
+                 35: 4, 36: fake, 37: 64}.items():
+        args[i] = v
+    assert fn(*args) == _lib.AKV_EINVAL
+    assert "aligned bytes" in _lib.last_error()
