@@ -8,18 +8,21 @@
 // which equals the reference's o * sigmoid(lse - sink)
 // (akv/system/sglang/srt/layers/attention/context_backend.py:254-272).
 //
-// Split-K: workgroup = one wave = (chunk of kChunk keys, KV head, request).
-// Per 16-key tile:  S^T[16 keys x 16 heads] = K[16 x D] . Q^T[D x 16] on
-// v_mfma_f32_16x16x16_bf16 (the group's q heads padded to 16 rows), online
-// softmax per head (column), then O^T[D x 16] += V^T[D x 16] . P^T[16 x 16]
-// where P^T is already in the B-operand layout of the second MFMA (no
-// shuffle) and V goes through LDS to be read transposed.  A combine kernel
-// merges the chunks and the sink; when every request fits one chunk (a
-// sliding-window layer) the partial kernel applies the sink itself and the
-// combine is not launched.
+// Split-K: workgroup = (chunk of keys, KV head, request), in passes of 256
+// keys: D / 16 waves of 4096 / D keys each.  A wave brings all its keys of a
+// pass at once -- slots, then K into registers in the operand layout and V
+// straight into its own LDS tile -- so a pass is two round trips, whatever its
+// length, and needs no barrier.  S^T[keys x 16 heads] = K . Q^T on
+// v_mfma_f32_16x16x32_bf16 (the group's q heads padded to 16), one softmax
+// step per pass, then O^T[D x 16] += V^T . P^T, where P^T is already in the
+// B-operand layout of the second MFMA (a lane's keys 4 (l/16) + i of two
+// 16-key tiles) and V^T comes from ds_read_b64_tr_b16.  The waves' results
+// meet in LDS at the end.  A combine kernel merges the chunks and the sink;
+// when every request fits one chunk (a sliding-window layer) the first kernel
+// applies the sink itself and the combine is not launched.
 //
-// MFMA 16x16x16 bf16 lane layout (verified on gfx950): lane l supplies
-// A[l%16][4(l/16)+i] and B[4(l/16)+i][l%16] and holds D[4(l/16)+i][l%16].
+// MFMA 16x16x32 bf16 lane layout (verified on gfx950): lane l supplies
+// A[l%16][k(l, i)] and B[k(l, i)][l%16], i < 8, and holds D[4(l/16)+i][l%16].
 #include <cmath>
 
 #include <mutex>
@@ -29,14 +32,17 @@
 namespace akv {
 namespace {
 
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) u32x4 global_u32x4;
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) void lds_void;
 
-constexpr int kChunk = 256;  // keys per workgroup
-constexpr int kTile = 16;    // keys per MFMA tile
+constexpr int kPass = 256;  // keys of a workgroup's pass
 constexpr float kLog2e = 1.4426950408889634f;
 
 struct AttnArgs {
@@ -54,215 +60,206 @@ struct AttnArgs {
   int32_t out_f32;
   int64_t out_stride_b, out_stride_h;
   int32_t n_requests, q_heads, kv_heads, group, chunks;
+  int32_t chunk_keys;  // keys per workgroup, a multiple of kPass
+  int32_t q_vectors;   // q rows are 16-byte aligned
   float* partial;  // [B][Hkv][chunks][16][D + 2]  (o..., m, l)
 };
 
-__device__ __forceinline__ short bf16_bits(float x) {
-  return __builtin_bit_cast(short, static_cast<__bf16>(x));
-}
+// The V rows of keys past a chunk's end: their weights are 0, and 0 times
+// whatever a real row holds (infinities) need not be 0.
+static __device__ __attribute__((aligned(16))) const uint32_t zero_row[64] = {};
 
-// Workgroup = one wave = (chunk of kChunk keys, KV head, request).  (Putting
-// all KV heads of a chunk in one workgroup, so key rows are read whole,
-// measured slower: the per-tile barrier then couples 8 waves.)
+// 16-byte chunk c of V row r sits at chunk c ^ swz(r) of its LDS row: distinct
+// bank groups for the 8 rows of a transposing read, a chunk pair stays adjacent.
 template <int D>
-__global__ void __launch_bounds__(64) decode_attention_partial_kernel(const AttnArgs a) {
-  constexpr int kSteps = D / 16;    // MFMA k-steps over the head dim
-  constexpr int kPer = D / 4;       // dims per lane for the K operand
-  __shared__ __attribute__((aligned(16))) __bf16 vtile[kTile][D];
+__device__ __forceinline__ int swz(int r) { return D == 64 ? r & 6 : (r & 7) << 1; }
 
-  const int lane = threadIdx.x;
-  const int chunk = blockIdx.x;
-  const int g = blockIdx.y;
-  const int b = blockIdx.z;
+// Bound by the HBM's random rows: 32 GPT-OSS requests of ~20k keys (1.29 GB)
+// take 245 us, 5.3 TB/s, where a large copy reaches 4.9 (read + write); with one
+// wave per 256 keys, 16 at a time, they took 256.  Four requests of 1-6k keys,
+// where the chain of round trips counts, take 11 us against 20; a 128-key
+// window 6-7 us against 12-13.  Grid: chunks fastest, so neighbouring
+// workgroups read different rows; a chunk's KV heads one after the other on
+// one XCD measured 4% slower (295 against 284 us for the decode step).
+template <int D>
+__global__ void __launch_bounds__(4 * D, 4) decode_attention_partial_kernel(const AttnArgs a) {
+  constexpr int kWaves = D / 16;
+  constexpr int kKeys = kPass / kWaves;       // keys of a wave's pass: 64 / 32
+  constexpr int kTiles = kKeys / 16;          // 16-key tiles
+  constexpr int kSteps = D / 32;              // MFMA k-steps over the head dim
+  constexpr int kDTiles = D / 16;
+  constexpr int kChunks = D / 8;              // 16-byte chunks of a row
+  constexpr int kRows = 64 / kChunks;         // V rows of one wave-wide load
+  constexpr int kOut = D + 4;                 // floats of an O row in LDS (padded: no bank conflicts)
+  constexpr int kWaveBytes = kKeys * D * 2 > 16 * kOut * 4 ? kKeys * D * 2 : 16 * kOut * 4;
+  __shared__ __attribute__((aligned(16))) char tiles[kWaves][kWaveBytes];
+  __shared__ float s_m[kWaves][16], s_l[kWaves][16];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int chunk = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
   const int64_t begin = a.kv_indptr[b];
   const int64_t len = a.kv_indptr[b + 1] - begin;
   // a closed gate stops the workgroup before its key indices and rows
   if (gated(a.gate)) return;
-  const int64_t c0 = static_cast<int64_t>(chunk) * kChunk;
-  float* part = a.partial + ((static_cast<int64_t>(b) * a.kv_heads + g) * a.chunks + chunk) * 16 * (D + 2);
+  const int64_t c0 = static_cast<int64_t>(chunk) * a.chunk_keys;
+  // an empty chunk is not read by the combine; with one chunk the output is 0
+  if (c0 >= len && a.chunks > 1) return;
+  const int n = static_cast<int>(len - c0 < a.chunk_keys ? (len > c0 ? len - c0 : 0) : a.chunk_keys);
+  const int32_t* idx = a.kv_indices + begin + c0;
   const int col = lane & 15;   // head within the group (B / D layout column)
   const int quad = lane >> 4;  // 0..3
-  if (c0 >= len) {
-    if (a.chunks == 1) {
-      // one chunk and no keys: the output is 0, sink or not (no combine runs)
-      if (col < a.group) {
-        const int64_t at = static_cast<int64_t>(b) * a.out_stride_b +
-                           static_cast<int64_t>(g * a.group + col) * a.out_stride_h;
-#pragma unroll
-        for (int t = 0; t < D / 16; ++t)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int d = 16 * t + 4 * quad + i;
-            if (a.out_f32)
-              static_cast<float*>(a.out)[at + d] = 0.f;
-            else
-              static_cast<__bf16*>(a.out)[at + d] = static_cast<__bf16>(0.f);
-          }
-      }
-      return;
-    }
-    // empty chunk: neutral partial (m = -inf, l = 0)
-    if (quad == 0) {
-      part[col * (D + 2) + D] = -INFINITY;
-      part[col * (D + 2) + D + 1] = 0.f;
-    }
-    return;
-  }
-  const int64_t c1 = c0 + kChunk < len ? c0 + kChunk : len;
 
-  // Q^T operand: lane supplies q[head col][dims quad*kPer + 4s + i]
-  s16x4 qop[kSteps];
+  // Q^T operand: lane supplies q[head col][dims 32 st + 8 quad + i]
+  bf16x8 qop[kSteps];
   {
-    const bool live = col < a.group;
+    // columns past the group repeat its last head; they are never stored
     const __bf16* qrow = a.q + static_cast<int64_t>(b) * a.q_stride_b +
-                         static_cast<int64_t>(g * a.group + (live ? col : 0)) * a.q_stride_h + quad * kPer;
-#pragma unroll
-    for (int s = 0; s < kSteps; ++s)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) qop[s][i] = live ? __builtin_bit_cast(short, qrow[4 * s + i]) : short(0);
-  }
-
-  f32x4 acc[D / 16];
-#pragma unroll
-  for (int t = 0; t < D / 16; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-
-  // Registers of one 16-key tile between its global loads and its use.
-  constexpr int kVUnits = kTile * D / 8 / 64;  // 16-byte V units per lane
-  struct Tile {
-    u32x4 k[kPer / 8];
-    u32x4 v[kVUnits];
-  };
-  auto load_tile = [&](int64_t t0) {
-    Tile r;
-    // this lane's key for the K operand / slot lookup: key t0 + col
-    const bool valid = t0 + col < c1;
-    const int32_t slot = valid ? a.kv_indices[begin + t0 + col] : 0;
-    const __bf16* krow =
-        a.k + static_cast<int64_t>(slot) * a.k_stride_slot + static_cast<int64_t>(g) * a.k_stride_head + quad * kPer;
-#pragma unroll
-    for (int q8 = 0; q8 < kPer / 8; ++q8)
-      r.k[q8] = valid ? *((const global_u32x4*)(krow + 8 * q8)) : u32x4{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int q8 = 0; q8 < kVUnits; ++q8) {
-      const int u = lane + 64 * q8;
-      const int key = u / (D / 8);
-      const int part8 = u - key * (D / 8);
-      const int32_t ks = __shfl(slot, key);
-      r.v[q8] = t0 + key < c1 ? *((const global_u32x4*)(a.v + static_cast<int64_t>(ks) * a.v_stride_slot +
-                                                        static_cast<int64_t>(g) * a.v_stride_head + part8 * 8))
-                              : u32x4{0u, 0u, 0u, 0u};
-    }
-    return r;
-  };
-
-  // Software-pipelined: the next tile's K and V loads are in flight while
-  // this tile's MFMAs and softmax run.
-  Tile cur = load_tile(c0);
-  for (int64_t t0 = c0; t0 < c1; t0 += kTile) {
-    Tile nxt = cur;
-    if (t0 + kTile < c1) nxt = load_tile(t0 + kTile);
-    // ---- S^T = K . Q^T
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
+                         static_cast<int64_t>(g * a.group + (col < a.group ? col : a.group - 1)) * a.q_stride_h + 8 * quad;
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) {
-      // dims quad*kPer + 4*st .. +3 live in k[st / 2], words (st % 2) * 2 .. +1
-      const u32x4 w = cur.k[st >> 1];
-      const uint32_t lo = (st & 1) ? w.z : w.x;
-      const uint32_t hi = (st & 1) ? w.w : w.y;
-      s16x4 kop;
-      kop[0] = static_cast<short>(lo & 0xffff);
-      kop[1] = static_cast<short>(lo >> 16);
-      kop[2] = static_cast<short>(hi & 0xffff);
-      kop[3] = static_cast<short>(hi >> 16);
-      s = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(kop, qop[st], s, 0, 0, 0);
-    }
-    // lane holds S^T[keys t0 + 4*quad + i][head col]
-    float p[4];
-    float tile_max = -INFINITY;
+      if (a.q_vectors) {
+        qop[st] = __builtin_bit_cast(bf16x8, *((const global_u32x4*)(qrow + 32 * st)));
+      } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const bool ok = t0 + 4 * quad + i < c1;
-      p[i] = ok ? s[i] * a.scale_log2 : -INFINITY;
-      tile_max = fmaxf(tile_max, p[i]);
+        for (int i = 0; i < 8; ++i) qop[st][i] = qrow[32 * st + i];
+      }
     }
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 16));
-    tile_max = fmaxf(tile_max, __shfl_xor(tile_max, 32));
-    const float m_new = fmaxf(m_run, tile_max);
+  }
+  const char* kbase = reinterpret_cast<const char*>(a.k + static_cast<int64_t>(g) * a.k_stride_head + 8 * quad);
+  const char* vbase = reinterpret_cast<const char*>(a.v + static_cast<int64_t>(g) * a.v_stride_head);
+  const int64_t k_slot = 2 * a.k_stride_slot, v_slot = 2 * a.v_stride_slot;
+
+  f32x4 acc[kDTiles];
+#pragma unroll
+  for (int t = 0; t < kDTiles; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  __bf16* vt = reinterpret_cast<__bf16*>(tiles[wave]);
+
+  for (int t0 = wave * kKeys; t0 < n; t0 += kPass) {
+    // this lane's key of the pass (keys past the end: the last one's row)
+    const int mine = t0 + (lane & (kKeys - 1));
+    const int32_t slot = idx[mine < n ? mine : n - 1];
+    u32x4 k[kTiles][kSteps];
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) {
+      const char* row = kbase + __shfl(slot, 16 * j + col) * k_slot;
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st) k[j][st] = *((const global_u32x4*)(row + 64 * st));
+    }
+#pragma unroll
+    for (int u = 0; u < kKeys / kRows; ++u) {
+      const int r = u * kRows + lane / kChunks;
+      const int c = (lane % kChunks) ^ swz<D>(r);
+      const char* row = vbase + __shfl(slot, r) * v_slot;
+      if (t0 + r >= n) row = reinterpret_cast<const char*>(zero_row);
+      __builtin_amdgcn_global_load_lds(row + 16 * c, (lds_void*)(vt + u * kRows * D), 16, 0, 0);
+    }
+    // ---- S^T = K . Q^T; lane holds S^T[keys 16 j + 4 quad + i][head col]
+    f32x4 p[kTiles];
+    float top = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < kTiles; ++j) {
+      f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int st = 0; st < kSteps; ++st)
+        s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, k[j][st]), qop[st], s, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[j][i] = t0 + 16 * j + 4 * quad + i < n ? s[i] * a.scale_log2 : -INFINITY;
+        top = fmaxf(top, p[j][i]);
+      }
+    }
+    top = fmaxf(top, __shfl_xor(top, 16));
+    top = fmaxf(top, __shfl_xor(top, 32));
+    const float m_new = fmaxf(m_run, top);
     const float corr = m_new == -INFINITY ? 1.f : exp2f(m_run - m_new);
     float row = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      p[i] = m_new == -INFINITY ? 0.f : exp2f(p[i] - m_new);
-      row += p[i];
-    }
+    for (int j = 0; j < kTiles; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        p[j][i] = m_new == -INFINITY ? 0.f : exp2f(p[j][i] - m_new);
+        row += p[j][i];
+      }
     row += __shfl_xor(row, 16);
     row += __shfl_xor(row, 32);
     l_run = l_run * corr + row;
     m_run = m_new;
 #pragma unroll
-    for (int t = 0; t < D / 16; ++t) acc[t] *= corr;
+    for (int t = 0; t < kDTiles; ++t) acc[t] *= corr;
+    // ---- O^T += V^T . P^T, once this wave's V rows have landed
+    __builtin_amdgcn_s_waitcnt(0);
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int jj = 0; jj < kTiles / 2; ++jj) {
+      const bf16x4 p0 = __builtin_convertvector(p[2 * jj], bf16x4), p1 = __builtin_convertvector(p[2 * jj + 1], bf16x4);
+      const bf16x8 pop = __builtin_shufflevector(p0, p1, 0, 1, 2, 3, 4, 5, 6, 7);
+      // transposing read: lane col of group quad receives V[key][16 t + col]
+      // for keys 32 jj + 4 quad + i, then 16 keys on; its source is row
+      // key0 + col / 4, dims 16 t + 4 (col % 4) .. + 3
+      const int r0 = 32 * jj + 4 * quad + (col >> 2), r1 = r0 + 16;
+#pragma unroll
+      for (int t = 0; t < kDTiles; ++t) {
+        const int c = 2 * t + ((col & 3) >> 1), h = 4 * (col & 1);
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vt + r0 * D + 8 * (c ^ swz<D>(r0)) + h));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(vt + r1 * D + 8 * (c ^ swz<D>(r1)) + h));
+        const bf16x8 vop = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop, acc[t], 0, 0, 0);
+      }
+    }
+    asm volatile("" ::: "memory");
+  }
 
-    // ---- V tile -> LDS (16 keys x D); rows past the chunk were loaded as 0
+  // the waves meet: O rows [head][dim] over their V tiles, m and l beside them
+  // (every lane of a column carries that head's m and l)
+  float* om = reinterpret_cast<float*>(tiles[wave]);
 #pragma unroll
-    for (int q8 = 0; q8 < kVUnits; ++q8) {
-      const int u = lane + 64 * q8;
-      const int key = u / (D / 8);
-      *reinterpret_cast<u32x4*>(&vtile[key][(u - key * (D / 8)) * 8]) = cur.v[q8];
-    }
-    __syncthreads();
-    // ---- O^T += V^T . P^T ; P^T is this lane's B operand as is
-    s16x4 pop;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) pop[i] = bf16_bits(p[i]);
-#pragma unroll
-    for (int t = 0; t < D / 16; ++t) {
-      s16x4 vop;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) vop[i] = __builtin_bit_cast(short, vtile[4 * quad + i][16 * t + col]);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(vop, pop, acc[t], 0, 0, 0);
-    }
-    __syncthreads();
-    cur = nxt;
+  for (int t = 0; t < kDTiles; ++t) *reinterpret_cast<f32x4*>(om + col * kOut + 16 * t + 4 * quad) = acc[t];
+  if (quad == 0) {
+    s_m[wave][col] = m_run;
+    s_l[wave][col] = l_run;
   }
-  // lane holds O^T[dims 16t + 4*quad + i][head col]; every lane of a column
-  // carries that head's m and l
-  if (a.chunks == 1) {
+  __syncthreads();
+  for (int u = threadIdx.x; u < a.group * (D / 4); u += 64 * kWaves) {
+    const int hl = u / (D / 4), d = 4 * (u % (D / 4));
+    float m = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) m = fmaxf(m, s_m[w][hl]);
+    float l = 0.f;
+    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      // a wave without keys carries m = -inf, l = 0 and O = 0
+      const float sw = s_m[w][hl] == -INFINITY ? 0.f : exp2f(s_m[w][hl] - m);
+      l += s_l[w][hl] * sw;
+      o += *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(tiles[w]) + hl * kOut + d) * sw;
+    }
+    if (a.chunks > 1) {
+      // a partial row is D + 2 floats: 8-byte aligned
+      float* ph = a.partial + (((static_cast<int64_t>(b) * a.kv_heads + g) * a.chunks + chunk) * 16 + hl) * (D + 2);
+      *reinterpret_cast<f32x2_t*>(ph + d) = f32x2_t{o[0], o[1]};
+      *reinterpret_cast<f32x2_t*>(ph + d + 2) = f32x2_t{o[2], o[3]};
+      if (d == 0) *reinterpret_cast<f32x2_t*>(ph + D) = f32x2_t{m, l};
+      continue;
+    }
     // one chunk holds every key: normalise with the sink here (the combine's
-    // arithmetic for a single partial) and skip the combine launch
-    if (col < a.group) {
-      const int h = g * a.group + col;
-      const float sink = a.sinks ? a.sinks[h] * kLog2e : -INFINITY;
-      const bool valid = m_run != -INFINITY;
-      const float mt = valid ? fmaxf(sink, m_run) : sink;
-      float lt = (a.sinks && mt != -INFINITY) ? exp2f(sink - mt) : 0.f;
-      const float sw = valid ? exp2f(m_run - mt) : 0.f;
-      lt += valid ? l_run * sw : 0.f;
-      const int64_t at = static_cast<int64_t>(b) * a.out_stride_b + static_cast<int64_t>(h) * a.out_stride_h;
+    // arithmetic for a single partial)
+    const int head = g * a.group + hl;
+    const float sink = a.sinks ? a.sinks[head] * kLog2e : -INFINITY;
+    const bool valid = m != -INFINITY;
+    const float mt = valid ? fmaxf(sink, m) : sink;
+    float lt = (a.sinks && mt != -INFINITY) ? exp2f(sink - mt) : 0.f;
+    const float sw = valid ? exp2f(m - mt) : 0.f;
+    lt += valid ? l * sw : 0.f;
+    const int64_t at = static_cast<int64_t>(b) * a.out_stride_b + static_cast<int64_t>(head) * a.out_stride_h + d;
 #pragma unroll
-      for (int t = 0; t < D / 16; ++t)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const float ot = valid ? acc[t][i] * sw : 0.f;
-          const float r = lt > 0.f ? ot / lt : 0.f;
-          const int d = 16 * t + 4 * quad + i;
-          if (a.out_f32)
-            static_cast<float*>(a.out)[at + d] = r;
-          else
-            static_cast<__bf16*>(a.out)[at + d] = static_cast<__bf16>(r);
-        }
-    }
-    return;
-  }
-  if (col < a.group) {
-    float* ph = part + col * (D + 2);
-#pragma unroll
-    for (int t = 0; t < D / 16; ++t)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ph[16 * t + 4 * quad + i] = acc[t][i];
-    if (quad == 0) {
-      ph[D] = m_run;
-      ph[D + 1] = l_run;
+    for (int i = 0; i < 4; ++i) {
+      const float r = lt > 0.f ? (valid ? o[i] * sw : 0.f) / lt : 0.f;
+      if (a.out_f32)
+        static_cast<float*>(a.out)[at + i] = r;
+      else
+        static_cast<__bf16*>(a.out)[at + i] = static_cast<__bf16>(r);
     }
   }
 }
@@ -290,7 +287,7 @@ __global__ void __launch_bounds__(kCombineThreads) decode_attention_combine_kern
   const int64_t len = a.kv_indptr[b + 1] - a.kv_indptr[b];
   if (gated(a.gate)) return;
   // keys past max_len (a caller error) are not read: the partials stop there
-  const int64_t want = (len + kChunk - 1) / kChunk;
+  const int64_t want = (len + a.chunk_keys - 1) / a.chunk_keys;
   const int used = static_cast<int>(want < a.chunks ? want : a.chunks);
   const float* base = a.partial + (static_cast<int64_t>(b) * a.kv_heads + g) * a.chunks * 16 * (D + 2);
   float m = -INFINITY, l = 0.f;
@@ -341,7 +338,21 @@ __global__ void __launch_bounds__(kCombineThreads) decode_attention_combine_kern
     static_cast<__bf16*>(a.out)[at] = static_cast<__bf16>(r);
 }
 
-int64_t chunks_for(int64_t max_len) { return max_len <= 0 ? 1 : (max_len + kChunk - 1) / kChunk; }
+int64_t chunks_for(int64_t max_len, int64_t keys) { return max_len <= 0 ? 1 : (max_len + keys - 1) / keys; }
+
+// Passes of a workgroup: up to four where that still leaves eight workgroups
+// per CU (a quarter of the partial results), and two keys' worth of passes
+// rather than a second launch for requests that then fit one chunk.
+constexpr int kMaxPasses = 4;
+constexpr int64_t kEnoughGroups = 8 * 256;
+int32_t chunk_keys_for(int64_t requests, int64_t kv_heads, int64_t max_len) {
+  int32_t passes = 1;
+  while (passes < kMaxPasses &&
+         requests * kv_heads * chunks_for(max_len, 2 * passes * kPass) >= kEnoughGroups)
+    passes *= 2;
+  if (passes == 1 && max_len <= 2 * kPass) passes = 2;
+  return passes * kPass;
+}
 
 // Split-K scratch of akv_decode_attention_noalloc: a file-scope device array,
 // one per GPU, held until the process ends.  Host code never passes the
@@ -383,7 +394,7 @@ extern "C" int64_t akv_decode_attention_workspace_bytes(int32_t n_requests, int3
                                                          int32_t head_dim, int64_t max_len) {
   using namespace akv;
   if (n_requests < 0 || kv_heads <= 0 || head_dim <= 0 || max_len < 0) return -1;
-  return static_cast<int64_t>(n_requests) * kv_heads * chunks_for(max_len) * 16 * (head_dim + 2) * 4;
+  return static_cast<int64_t>(n_requests) * kv_heads * chunks_for(max_len, kPass) * 16 * (head_dim + 2) * 4;
 }
 
 extern "C" int akv_decode_attention(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* k_buffer,
@@ -438,25 +449,24 @@ extern "C" int akv_decode_attention(const void* q, int64_t q_stride_b, int64_t q
   a.q_heads = q_heads;
   a.kv_heads = kv_heads;
   a.group = q_heads / kv_heads;
-  a.chunks = static_cast<int32_t>(chunks_for(max_len));
+  a.chunk_keys = chunk_keys_for(n_requests, kv_heads, max_len);
+  a.chunks = static_cast<int32_t>(chunks_for(max_len, a.chunk_keys));
+  a.q_vectors = ((q_stride_b | q_stride_h) % 8 == 0) && (reinterpret_cast<uintptr_t>(q) & 15) == 0;
   a.partial = static_cast<float*>(workspace);
   hipStream_t st = as_stream(stream);
   const dim3 grid(static_cast<unsigned>(a.chunks), static_cast<unsigned>(kv_heads),
                   static_cast<unsigned>(n_requests));
-  const dim3 block(64);
-  if (head_dim == 64) {
-    hipLaunchKernelGGL(decode_attention_partial_kernel<64>, grid, block, 0, st, a);
-    int rc = check_launch("akv_decode_attention (partial)");
-    if (rc || a.chunks == 1) return rc;
-    hipLaunchKernelGGL(decode_attention_combine_kernel<64>, dim3(n_requests, q_heads), dim3(kCombineThreads), 0,
-                       st, a);
-  } else {
-    hipLaunchKernelGGL(decode_attention_partial_kernel<128>, grid, block, 0, st, a);
-    int rc = check_launch("akv_decode_attention (partial)");
-    if (rc || a.chunks == 1) return rc;
-    hipLaunchKernelGGL(decode_attention_combine_kernel<128>, dim3(n_requests, q_heads), dim3(kCombineThreads), 0,
-                       st, a);
-  }
+  if (head_dim == 64)
+    hipLaunchKernelGGL(decode_attention_partial_kernel<64>, grid, dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(decode_attention_partial_kernel<128>, grid, dim3(512), 0, st, a);
+  int rc = check_launch("akv_decode_attention (partial)");
+  if (rc || a.chunks == 1) return rc;
+  const dim3 merge(n_requests, q_heads);
+  if (head_dim == 64)
+    hipLaunchKernelGGL(decode_attention_combine_kernel<64>, merge, dim3(kCombineThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL(decode_attention_combine_kernel<128>, merge, dim3(kCombineThreads), 0, st, a);
   return check_launch("akv_decode_attention (combine)");
 }
 
