@@ -92,8 +92,13 @@ struct WindowArgs {
   bool rows64, lengths64, output64;
 };
 
-__global__ void __launch_bounds__(256) window_lengths_kernel(const WindowArgs a) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+// One wave per request: its lanes probe the positions together (three rounds
+// of loads for 20k keys, where a binary search takes fifteen).
+constexpr int kWindowRequests = 4;  // requests (waves) per workgroup
+
+__global__ void __launch_bounds__(64 * kWindowRequests) window_lengths_kernel(const WindowArgs a) {
+  const int b = blockIdx.x * kWindowRequests + static_cast<int>(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
   if (b >= a.n_requests) return;
   const int64_t row = load_index(a.rows, a.rows64, b);
   const int64_t length = load_index(a.lengths, a.lengths64, b);
@@ -106,17 +111,11 @@ __global__ void __launch_bounds__(256) window_lengths_kernel(const WindowArgs a)
     const int64_t generated = length - active;
     // visible keys satisfy q_pos - k_pos <= window (inclusive)
     const int64_t lower = next_pos + generated - 1 - a.window;
-    int32_t lo = 0, hi = active;
-    while (lo < hi) {
-      const int32_t mid = lo + ((hi - lo) >> 1);
-      if (positions[mid] < lower)
-        lo = mid + 1;
-      else
-        hi = mid;
-    }
+    const int32_t lo = first_at_least([&](int32_t i) -> int64_t { return positions[i]; }, active, lower, lane);
     const int64_t skipped = lower - next_pos > 0 ? lower - next_pos : 0;
     result = active - lo + generated - skipped;
   }
+  if (lane != 0) return;
   store_index(a.output, a.output64, b, result);
   if (a.starts) store_index(a.starts, a.lengths64, b, length - result);
 }
@@ -131,7 +130,7 @@ struct IndptrArgs {
   bool lengths64, indptr64;
 };
 
-// One workgroup: exclusive scan of the request lengths.
+// One workgroup, no wider than the batch: exclusive scan of the request lengths.
 __global__ void __launch_bounds__(1024) build_indptr_kernel(const IndptrArgs a) {
   __shared__ int64_t wave_tot[16];
   __shared__ int64_t carry;
@@ -297,7 +296,8 @@ extern "C" int akv_window_lengths(const int64_t* registry, const void* rows, int
   a.rows64 = rows_dtype == AKV_I64;
   a.lengths64 = lengths_dtype == AKV_I64;
   a.output64 = output_dtype == AKV_I64;
-  hipLaunchKernelGGL(window_lengths_kernel, dim3((n_requests + 255) / 256), dim3(256), 0, as_stream(stream), a);
+  hipLaunchKernelGGL(window_lengths_kernel, dim3((n_requests + kWindowRequests - 1) / kWindowRequests),
+                     dim3(64 * kWindowRequests), 0, as_stream(stream), a);
   return check_launch("akv_window_lengths");
 }
 
@@ -320,7 +320,8 @@ extern "C" int akv_build_indptr(const void* lengths, int32_t lengths_dtype, int3
   a.page_size = page_size;
   a.lengths64 = lengths_dtype == AKV_I64;
   a.indptr64 = indptr_dtype == AKV_I64;
-  hipLaunchKernelGGL(build_indptr_kernel, dim3(1), dim3(1024), 0, as_stream(stream), a);
+  const unsigned threads = n_requests >= 1024 ? 1024u : n_requests <= 64 ? 64u : (n_requests + 63u) / 64u * 64u;
+  hipLaunchKernelGGL(build_indptr_kernel, dim3(1), dim3(threads), 0, as_stream(stream), a);
   return check_launch("akv_build_indptr");
 }
 
