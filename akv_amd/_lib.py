@@ -151,6 +151,7 @@ EXPORTED = tuple(_SIGNATURES)
 
 _lock = threading.Lock()
 _lib = None
+_calls = None
 
 
 class AkvError(RuntimeError):
@@ -176,6 +177,27 @@ def load():
                 fn.argtypes = argtypes
             _lib = lib
     return _lib
+
+
+def calls():
+    """The entry points the wrappers call per step, with native argument
+    conversion (``csrc/native.cpp``); same arguments and results as
+    ``load()``'s functions."""
+    global _calls
+    if _calls is not None:
+        return _calls
+    lib = load()
+    try:
+        from . import _native
+    except ImportError as e:
+        raise RuntimeError("akv_amd native calls not built (_native.so); run `python -m akv_amd.build`") from e
+    with _lock:
+        if _calls is None:
+            for name in _native.names():
+                fn = getattr(lib, name)
+                _native.bind(name, ctypes.cast(fn, c_void_p).value, fn)
+            _calls = _native
+    return _calls
 
 
 def last_error():

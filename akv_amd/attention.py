@@ -15,7 +15,7 @@ from .ops import _on_device, current_stream_handle
 
 
 def workspace_bytes(n_requests, kv_heads, head_dim, max_len):
-    return _lib.load().akv_decode_attention_workspace_bytes(n_requests, kv_heads, head_dim, max_len)
+    return _lib.calls().akv_decode_attention_workspace_bytes(n_requests, kv_heads, head_dim, max_len)
 
 
 def decode_attention(q, k_buffer, v_buffer, kv_indptr, kv_indices, out, *, scale, max_len, sinks=None,
@@ -50,7 +50,7 @@ def decode_attention(q, k_buffer, v_buffer, kv_indptr, kv_indices, out, *, scale
     need = workspace_bytes(n, hkv, d, max_len)
     if workspace is None:
         workspace = torch.empty(max(4, (need + 3) // 4), dtype=torch.float32, device=q.device)
-    lib = _lib.load()
+    lib = _lib.calls()
     with _on_device(q.device):
         rc = lib.akv_decode_attention(
             q.data_ptr(), q.stride(0), q.stride(1), k_buffer.data_ptr(), v_buffer.data_ptr(),

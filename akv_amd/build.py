@@ -1,7 +1,8 @@
 """Builds ``akv_amd/libakv_amd.so`` for gfx950 with hipcc (no GPU needed).
 
 Every translation unit is compiled to an object under ``akv_amd/_build/``
-in parallel, then linked into one shared library next to this file.  Device
+in parallel, then linked into one shared library next to this file, beside
+``_native.so``, the extension module through which Python calls it.  Device
 code is compiled with ``-ffp-contract=off`` (the Reposition arithmetic must
 round every product and sum separately) and without the packed-fp32
 instructions.
@@ -13,6 +14,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
@@ -20,6 +22,7 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 OUT_DIR = HERE / "_build"
 LIBRARY = HERE / "libakv_amd.so"
+NATIVE = HERE / "_native.so"
 ARCH = "gfx950"
 
 HIP_SOURCES = [
@@ -71,6 +74,10 @@ def build(verbose=False):
     tmp = LIBRARY.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", str(tmp)])
     os.replace(tmp, LIBRARY)
+    tmp = NATIVE.with_suffix(".so.tmp")
+    _run([hipcc, *COMMON_FLAGS, "-x", "c++", "-shared", "-I" + sysconfig.get_paths()["include"],
+          str(CSRC / "native.cpp"), "-o", str(tmp)])
+    os.replace(tmp, NATIVE)
     return LIBRARY
 
 

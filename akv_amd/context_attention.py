@@ -80,7 +80,7 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
     scale = sm_scale if sm_scale is not None else d ** -0.5
     if sinks is not None and (sinks.dtype != torch.float32 or sinks.shape != (q_extend.shape[1],)):
         raise ValueError("sinks must be f32 [q_heads]")
-    lib = _lib.load()
+    lib = _lib.calls()
     pos_dtype = _INDEX[context_q_positions.dtype] if use_context_positions else _lib.AKV_I64
     window = int(sliding_window_size) if sliding_window_size is not None else -1
     with _on_device(q_extend.device):

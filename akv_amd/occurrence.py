@@ -261,7 +261,7 @@ def bind_final_forward(inputs, req_to_token, req_rows, birth_slots, fresh_slots,
         raise ValueError("birth_slots must be int32 with one slot per raw token")
     if fresh_slots.dtype != torch.int32 or fresh_slots.shape != (sum(inputs.extra),):
         raise ValueError("Context admission does not cover the selected window")
-    lib = _lib.load()
+    lib = _lib.calls()
     device = req_to_token.device
     with _on_device(device):
         rc = lib.akv_bind_occurrences(

@@ -17,7 +17,8 @@ _KV_DTYPES = {torch.float32: _lib.AKV_F32, torch.float16: _lib.AKV_F16, torch.bf
 
 def current_stream_handle(device):
     """hipStream_t of torch's current stream on ``device``, as an int."""
-    return torch.cuda.current_stream(device).cuda_stream
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)  # no Stream object around the handle
 
 
 class _on_device:
@@ -30,7 +31,7 @@ class _on_device:
         self.previous = None
 
     def __enter__(self):
-        current = torch.cuda.current_device()
+        current = torch._C._cuda_getDevice()  # the caller's tensors are on a device: nothing to initialise
         if current != self.index:
             self.previous = current
             torch.cuda.set_device(self.index)
@@ -166,7 +167,7 @@ def _reposition(k_data_ptrs, v_data_ptrs, k_layout, v_layout, source_slots, dest
     table_dtype = _KV_DTYPES.get(cos_sin_cache.dtype)
     if table_dtype is None:
         raise ValueError("Reposition cos/sin cache must be float32, float16 or bfloat16")
-    lib = _lib.load()
+    lib = _lib.calls()
     with _on_device(k_layout.device):
         rc = lib.akv_reposition_kv_layers_gated(
             k_data_ptrs.data_ptr(),

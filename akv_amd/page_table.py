@@ -60,7 +60,7 @@ def context_decode_indices(registry, table, rows, lengths, indptr, output, *, st
     map_p, map_t = _idx(mapping, "mapping")
     device = output.device
     with _on_device(device):
-        rc = _lib.load().akv_decode_indices(
+        rc = _lib.calls().akv_decode_indices(
             registry.data_ptr(), table.data_ptr(), table.stride(0), rows_p, rows_t, len_p, len_t,
             ind_p, ind_t, out_p, out_t, st_p, st_t, map_p, map_t, int(multiplier), len(lengths),
             _status_ptr(status, device), current_stream_handle(device),
@@ -77,7 +77,7 @@ def context_window_lengths(registry, rows, lengths, output, window, *, starts=No
         raise ValueError("starts must have the dtype of lengths")
     device = output.device
     with _on_device(device):
-        rc = _lib.load().akv_window_lengths(
+        rc = _lib.calls().akv_window_lengths(
             registry.data_ptr(), rows_p, rows_t, len_p, len_t, out_p, out_t, _lib.ptr(starts),
             int(window), len(lengths), current_stream_handle(device),
         )
@@ -92,7 +92,7 @@ def build_indptr(lengths, indptr, *, last_page_len=None, page_size=1):
         raise ValueError("last_page_len must be int32")
     device = indptr.device
     with _on_device(device):
-        rc = _lib.load().akv_build_indptr(
+        rc = _lib.calls().akv_build_indptr(
             len_p, len_t, len(lengths), ind_p, ind_t, _lib.ptr(last_page_len), int(page_size), 1,
             current_stream_handle(device),
         )
@@ -107,7 +107,7 @@ def table_indptr(batch, stride, indptr):
         raise ValueError("table_indptr needs a row stride other than 1")
     device = indptr.device
     with _on_device(device):
-        rc = _lib.load().akv_build_indptr(
+        rc = _lib.calls().akv_build_indptr(
             None, _lib.AKV_I32, batch, ind_p, ind_t, None, 1, int(stride), current_stream_handle(device)
         )
     _lib.check(rc, "akv_build_indptr")
@@ -122,7 +122,7 @@ def write_row_slots(pointers, rows, columns, values):
     val_p, val_t = _idx(values, "values")
     device = pointers.device
     with _on_device(device):
-        rc = _lib.load().akv_write_row_slots(
+        rc = _lib.calls().akv_write_row_slots(
             pointers.data_ptr(), rows_p, rows_t, col_p, col_t, val_p, val_t, rows.numel(),
             current_stream_handle(device),
         )
@@ -154,7 +154,7 @@ def write_req_to_token_pool(req_to_token, req_pool_indices, prefix_tensors, pre_
         raise ValueError("prefix_dtype must be int32 or int64")
     device = req_to_token.device
     with _on_device(device):
-        rc = _lib.load().akv_write_extend_rows(
+        rc = _lib.calls().akv_write_extend_rows(
             req_to_token.data_ptr(), req_to_token.stride(0), _lib.ptr(row_pointers), rows_p, rows_t,
             prefix_tensors.data_ptr(), prefix_t, pre_lens.data_ptr(), seq_lens.data_ptr(), extend_lens.data_ptr(),
             len_t, loc_p, loc_t, len(req_pool_indices), current_stream_handle(device),

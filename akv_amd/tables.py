@@ -178,7 +178,7 @@ def compact_rows(inputs, req_to_token, req_rows, fresh_slots, outputs, *, row_po
         raise ValueError("generated entries need kv_indices outputs")
     if row_pointers is None and req_to_token.shape[1] < inputs.max_tokens:
         raise ValueError("req_to_token rows are shorter than the longest request")
-    lib = _lib.load()
+    lib = _lib.calls()
     device = req_to_token.device
     with _on_device(device):
         rc = lib.akv_compact_rows(
@@ -403,7 +403,7 @@ def compact_pages(inputs, req_to_token, req_rows, fresh_pages, outputs, *, row_p
         t = getattr(outputs, name)
         if t.dtype != torch.int32 or tuple(t.shape) != shape or not t.is_contiguous():
             raise ValueError(f"outputs.{name} must be a contiguous int32 tensor of shape {shape}")
-    lib = _lib.load()
+    lib = _lib.calls()
     device = req_to_token.device
     # an empty list (a batch with nothing copied or released) gets a valid
     # one-element stand-in: the kernel's writes to it are bounded by a zero total

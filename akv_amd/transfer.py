@@ -55,7 +55,7 @@ def copy_kv_rows(src_k_ptrs, src_v_ptrs, src_layout, dst_k_ptrs, dst_v_ptrs, dst
     if status is not None and (status.dtype != torch.int32 or status.numel() < 1
                                or status.device != src_k_ptrs.device):
         raise ValueError("status must be an int32 device word on the pointer tables' device")
-    lib = _lib.load()
+    lib = _lib.calls()
     device = src_k_ptrs.device
     with _on_device(device):
         rc = lib.akv_copy_kv_rows(
