@@ -519,13 +519,19 @@ __global__ void __launch_bounds__(256) reposition_generic_kernel(const Repositio
 // rule: about 256 threads of consecutive tokens, one layer each.
 // The sweep order, measured on MI355X: every layer's workgroup re-reads its
 // tokens' cos/sin rows (25% over the K/V reads of a GPT-OSS row), which
-// stays cheap while the rows of all tokens stay cached.  So one sweep when
-// they fit kSweepTableBytes (the 32k GPT-OSS request's 12064 copies: 6 MB;
-// chunks of 4096-12288 tokens measured 0.5-1.5% slower), else chunks of
-// kChunkTokens tokens, each swept over every layer before the next (Llama-3
-// page-16 copy-on-write, 777k copies and 777 MB of table rows: 61% of HBM
+// stays cheap while the rows of all tokens stay cached.  One sweep then also
+// reads source rows that several requests share (page-16 copy-on-write of a
+// common prefix) while a layer's rows are still cached.  So one sweep when the
+// table rows fit kSweepTableBytes, well inside the 256 MB last-level cache:
+// four Llama-3 requests over a shared 8k prefix, 43k copies and 44 MB of table
+// rows, 1946 us against 2227 in chunks; distinct positions, Llama-3 rows of 16
+// layers, sweep | chunks of 1024: 26 MB 647 | 660 us, 51 MB 1170-1300 | 1310,
+// 102 MB 2411-2707 | 2636, 154 MB 4082 | 3244.  The 32k GPT-OSS request's
+// 12064 copies have 6 MB (chunks of 4096-12288 tokens measured 0.5-1.5%
+// slower).  Above, chunks of kChunkTokens tokens, each swept over every layer
+// before the next (777k Llama-3 copies and 777 MB of table rows: 61% of HBM
 // peak in one sweep, 72 / 75 / 76.7% in chunks of 16384 / 4096 / 1024).
-constexpr int64_t kSweepTableBytes = 16ll << 20;
+constexpr int64_t kSweepTableBytes = 64ll << 20;
 constexpr int64_t kChunkTokens = 1024;
 void geometry(RepositionArgs& a) {
   int tokens = 256 / a.lanes_per_row;
