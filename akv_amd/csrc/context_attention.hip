@@ -735,7 +735,10 @@ __device__ __forceinline__ void attend(const CtxArgs& a, const Lds<D, KEYS, SUB>
           oacc[dt][s] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[s], oacc[dt][s], 0, 0, 0);
       }
     };
-    if constexpr (SPLIT) {
+    if constexpr (SPLIT && kKeys == 64) {
+      if (share == 0) half(0);
+      if (sharers == 1 || share == 1) half(1);
+    } else if constexpr (SPLIT) {
 #pragma nounroll
       for (int kk = share; kk < kKeys / 32; kk += sharers) half(kk);
     } else if constexpr (kKeys == 64) {
