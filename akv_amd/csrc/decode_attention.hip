@@ -75,9 +75,9 @@ template <int D>
 __device__ __forceinline__ int swz(int r) { return D == 64 ? r & 6 : (r & 7) << 1; }
 
 // Bound by the HBM's random rows: 32 GPT-OSS requests of ~20k keys (1.29 GB)
-// take 245 us, 5.3 TB/s, where a large copy reaches 4.9 (read + write); with one
+// take 247 us, 5.2 TB/s, where a large copy reaches 4.9 (read + write); with one
 // wave per 256 keys, 16 at a time, they took 256.  Four requests of 1-6k keys,
-// where the chain of round trips counts, take 11 us against 20; a 128-key
+// where the chain of round trips counts, take 10 us against 20; a 128-key
 // window 6-7 us against 12-13.  Grid: chunks fastest, so neighbouring
 // workgroups read different rows; a chunk's KV heads one after the other on
 // one XCD measured 4% slower (295 against 284 us for the decode step).
