@@ -20,7 +20,7 @@
 // fastest in the grid (workgroup id mod 8 picks the XCD: with 8 KV heads each
 // XCD's L2 serves one head's K/V), with the
 // G q heads of the group packed as rows: row r = token * G + head; R = 512
-// rows at head_dim 64 (8 waves x 64 rows, so each wave's reads of a K/V tile
+// rows at head_dim 64 (8 waves x 64 rows, 16 for narrow windows; a wave's reads of a K/V tile
 // from LDS feed 64 rows), 256 at head_dim 128 (8 waves x 32 rows); one
 // workgroup per CU, two waves per SIMD, so every K/V tile a CU stages from
 // L2 feeds all of its rows.  Per
@@ -46,6 +46,10 @@
 // lane l uses keys 4(l/16)+i of two 16-key subtiles); V^T comes from the
 // key-major tile through ds_read_b64_tr_b16.  Tiles wholly inside every
 // row's causal and window range skip the mask.
+//
+// Batches whose plain grid leaves CUs idle take the split launch: one
+// workgroup per CU with an equal stretch of all key tiles (context_plan.h), and
+// a second launch that merges the blocks a stretch boundary cut.
 //
 // Two instances of each shape: the plain one (head_dim 64 or 128, the group
 // a power of two, no logit cap) and the general one, which pads a token's
@@ -740,7 +744,8 @@ __device__ __forceinline__ void attend(const CtxArgs& a, const Lds<D, KEYS, SUB>
       if (sharers == 1 || share == 1) half(1);
     } else if constexpr (SPLIT) {
 #pragma nounroll
-      for (int kk = share; kk < kKeys / 32; kk += sharers) half(kk);
+      for (int kk = 0; kk < kKeys / 32; ++kk)
+        if ((kk & (sharers - 1)) == share) half(kk);
     } else if constexpr (kKeys == 64) {
       half(0);
       half(1);
@@ -983,13 +988,13 @@ __global__ void __launch_bounds__(kThreads, 2) context_split_kernel(const CtxArg
 // Workgroup = (64 / 32 rows of one wave of the main kernel, boundary); the
 // block's first boundary does the work.  A wave takes one row subtile and two
 // 16-dim tiles, every lane the same rows and dims as in the main kernel, so
-// the parts are read in whole 1 KiB accesses, eight parts at a time: the cost
+// the parts are read in whole 1 KiB accesses, four parts at a time: the cost
 // is round trips (the cuts, then the parts), not bandwidth.
 constexpr int kCombineDims = 2;  // 16-dim tiles of a wave
 template <int D, bool GEN>
 __global__ void __launch_bounds__(512) context_combine_kernel(const CtxArgs a) {
   constexpr int kSub = sub_tiles(D);
-  constexpr int kAhead = 8;  // parts whose loads are in flight together
+  constexpr int kAhead = 4;  // parts in flight together (8 and 12: most blocks have fewer, 1-6% slower)
   static_assert(64 * kSub * (D / 16 / kCombineDims) == 512, "one wave per row subtile and pair of dim tiles");
   const int lane = threadIdx.x & 63;
   const int w = uniform(threadIdx.x >> 6);

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from akv_amd import _lib
+from akv_amd import _lib, context_attention as ca
 from test_gpu_context_attention import TOL, _case, _run
 
 pytestmark = pytest.mark.gpu
@@ -66,6 +66,50 @@ def test_split_parts_far_apart(device, d, hq, hkv, step):
     got, want = _run(device, c, window=-1, positions=False, sinks=None, out_dtype=torch.float32, scale=d ** -0.5)
     assert np.isfinite(got).all()
     assert np.abs(got - want).max() <= TOL
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("idx,ind,pos", [(torch.int32, torch.int64, torch.int64), (torch.int64, torch.int32, torch.int32),
+                                         (torch.int64, torch.int64, None)])
+@pytest.mark.parametrize("segments", [1, 7, 64])
+def test_split_matches_plain(device, monkeypatch, d, idx, ind, pos, segments):
+    """The split launch against the plain one over index and position types,
+    strided queries, K/V, pools and outputs, and up to 64 segments (the last
+    lane of its plan); the two differ by the rounding of their sums."""
+    rng = np.random.default_rng(segments + d)
+    q_lens = rng.integers(0, 90, segments)
+    q_lens[0] = 37
+    p_lens = rng.integers(0, 300, segments) + (4000 // segments)
+    hq, hkv, nq, slots = 16, 2, int(q_lens.sum()), int(p_lens.sum()) + 8
+    g = torch.Generator().manual_seed(d)
+
+    def strided(n, heads):  # a view into wider rows
+        t = torch.randn((n, heads + 1, d), generator=g).to(torch.bfloat16).to(device)
+        return t[:, 1:]
+
+    q, ke, ve, kp, vp = strided(nq, hq), strided(nq, hkv), strided(nq, hkv), strided(slots, hkv), strided(slots, hkv)
+    indices = torch.from_numpy(rng.permutation(slots - 1)[: p_lens.sum()] + 1).to(idx).to(device)
+    qo = torch.from_numpy(np.concatenate(([0], np.cumsum(q_lens)))).to(ind).to(device)
+    kv = torch.from_numpy(np.concatenate(([0], np.cumsum(p_lens)))).to(ind).to(device)
+    qp = kpos = None
+    if pos is not None:
+        qp = torch.arange(nq, dtype=pos, device=device) + 100000
+        kpos = torch.arange(int(p_lens.sum()), dtype=pos, device=device)
+    workspace = torch.empty(70 << 20, dtype=torch.uint8, device=device)  # more than either head_dim needs
+
+    def run(split):
+        monkeypatch.setattr(ca, "_split_workspace", lambda *a: workspace if split else None)
+        out = torch.full((nq, hq + 2, d), 7.0, dtype=torch.float32, device=device)
+        ca.extend_attention_fwd(q, ke, ve, out[:, 1:-1], kp, vp, qo, kv, indices, None, True, None, int(q_lens.max()),
+                                context_q_positions=qp, context_kv_positions=kpos)
+        torch.cuda.synchronize()
+        assert (out[:, 0] == 7).all() and (out[:, -1] == 7).all()
+        return out[:, 1:-1]
+
+    got, want = run(True), run(False)
+    # both round the weights to bf16 (2^-9) against a different maximum, so an
+    # output differs by at most 2 x 2^-9 of the values' size (below 5)
+    assert (got - want).abs().max() <= 2e-2
 
 
 @pytest.mark.parametrize("positions", [True, False])
