@@ -66,6 +66,7 @@
 
 #include "common.h"
 #include "context_plan.h"
+#include "tile_loop.h"
 
 namespace akv {
 namespace {
@@ -327,7 +328,7 @@ struct Lds {
   TileLds<D, KEYS>& tile0;
   TileLds<D, KEYS>& tile1;
   int32_t (&rel_rows)[block_rows(SUB)];
-  int32_t& restart_flag;
+  int32_t (&restart)[kRestartWords];  // tile_loop.h
   float2* merge;  // 4 x 16 SUB, split launch only
 };
 
@@ -581,7 +582,7 @@ __device__ __forceinline__ void attend(const CtxArgs& a, const Lds<D, KEYS, SUB>
   bool unset = true;
   // after a restart every tile takes the exact maxima (uniform)
   bool exact_all = false;
-  if (tid == 0) lds.restart_flag = 0;
+  if (tid < kRestartWords) lds.restart[tid] = 0;
   const bf16x8 kOnes = {__bf16(1.f), __bf16(1.f), __bf16(1.f), __bf16(1.f),
                         __bf16(1.f), __bf16(1.f), __bf16(1.f), __bf16(1.f)};
 
@@ -768,7 +769,7 @@ __device__ __forceinline__ void attend(const CtxArgs& a, const Lds<D, KEYS, SUB>
       huge |= lacc[s][0] > kHuge;
     }
     if (__builtin_amdgcn_ballot_w64(big)) {
-      if (!exact && __builtin_amdgcn_ballot_w64(huge)) lds.restart_flag = 1;
+      if (!exact && __builtin_amdgcn_ballot_w64(huge)) lds.restart[restart_word(it_begin, it)] = 1;
       // sum -> [1/2, 1): O and the sum by 2^-e, the maximum up by e
 #pragma unroll
       for (int s = 0; s < kSub; ++s) {
@@ -791,27 +792,27 @@ __device__ __forceinline__ void attend(const CtxArgs& a, const Lds<D, KEYS, SUB>
     if (it + 1 < it_end) commit(nxt);
     __syncthreads();
   };
-  // a restart (decided before the tile's barrier, read after it by every
-  // wave) starts the keys again from tile 0 with exact maxima; no load is in
-  // flight after a barrier and neither buffer is still being read
-  auto restart_flag_set = [&]() -> bool {
-    return !exact_all && __builtin_amdgcn_readfirstlane(*static_cast<volatile int32_t*>(&lds.restart_flag));
-  };
-  auto restarted = [&]() -> bool {
-    if (!restart_flag_set()) return false;
-    exact_all = true;
-    unset = true;
-    clear_rows();
-    if (it_begin < n_pref) fetch_slots(it_begin);
-    open();
-    return true;
-  };
-  for (int it = it_begin; it < it_end; it += 2) {
-    step(it, lds.tile0, lds.tile1);
-    // a restart after the first half skips the second
-    if (it + 1 < it_end && !restart_flag_set()) step(it + 1, lds.tile1, lds.tile0);
-    if (restarted()) it = it_begin - 2;
-  }
+  // a restart starts the keys again from tile 0 with exact maxima; no load is
+  // in flight after a barrier and neither buffer is still being read
+  run_tiles(
+      it_begin, it_end,
+      [&](int it, auto half) {
+        if constexpr (half == 0)
+          step(it, lds.tile0, lds.tile1);
+        else
+          step(it, lds.tile1, lds.tile0);
+      },
+      [&](int it) -> bool {
+        const volatile int32_t* word = &lds.restart[restart_word(it_begin, it)];
+        return !exact_all && __builtin_amdgcn_readfirstlane(*word);
+      },
+      [&]() {
+        exact_all = true;
+        unset = true;
+        clear_rows();
+        if (it_begin < n_pref) fetch_slots(it_begin);
+        open();
+      });
 
   if constexpr (SPLIT) {
     // merge the sharers of each row group through the tiles' LDS (free after
@@ -880,8 +881,8 @@ template <int D, int KEYS, int SUB, typename IdxT, typename PosT, bool POS, bool
 __global__ void __launch_bounds__(kThreads, SUB == 1 ? 4 : 2) context_attention_kernel(const CtxArgs a) {
   __shared__ __attribute__((aligned(16))) TileLds<D, KEYS> tile0, tile1;
   __shared__ int32_t rel_rows[block_rows(SUB)];
-  __shared__ int32_t restart_flag;
-  const Lds<D, KEYS, SUB> lds{tile0, tile1, rel_rows, restart_flag, nullptr};
+  __shared__ int32_t restart[kRestartWords];
+  const Lds<D, KEYS, SUB> lds{tile0, tile1, rel_rows, restart, nullptr};
   // KV head fastest: workgroup id mod 8 picks the XCD, so with 8 KV heads
   // every XCD streams one head's K/V through its own L2.  Token blocks run
   // last-first: the last blocks see the most causal keys, and starting them
@@ -921,11 +922,11 @@ template <int D, int KEYS, typename IdxT, bool GEN>
 __global__ void __launch_bounds__(kThreads, 2) context_split_kernel(const CtxArgs args) {
   __shared__ __attribute__((aligned(16))) TileLds<D, KEYS> tile0, tile1;
   __shared__ int32_t rel_rows[rows_per_block(D)];
-  __shared__ int32_t restart_flag;
+  __shared__ int32_t restart[kRestartWords];
   __shared__ float2 merge[4 * 16 * sub_tiles(D)];
   __shared__ SplitState state;
   __shared__ int4 segments[kMaxSplitSegments];  // first query and prefix index, queries, prefix keys
-  const Lds<D, KEYS, sub_tiles(D)> lds{tile0, tile1, rel_rows, restart_flag, merge};
+  const Lds<D, KEYS, sub_tiles(D)> lds{tile0, tile1, rel_rows, restart, merge};
   {
     const SplitShape shape = split_shape<D, KEYS>(args);
     const int lane = threadIdx.x & 63;
