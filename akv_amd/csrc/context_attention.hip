@@ -209,10 +209,10 @@ constexpr int kMaxSplitSegments = 64;
 
 // One wave's copy of the batch: lane s holds segment s.
 struct BatchPlan {
-  int32_t q0, k0;  // this lane's segment: first query, first prefix index
+  int64_t q0, k0;  // this lane's segment: first query, first prefix index
   int32_t q, p;    // queries and prefix keys
-  int32_t before;  // cost of the segments before it
-  int32_t total;   // one head's cost
+  int64_t before;  // cost of the segments before it
+  int64_t total;   // one head's cost
   uint64_t live;   // segments with queries
 };
 
@@ -221,40 +221,51 @@ __device__ __forceinline__ SplitShape split_shape(const CtxArgs& a) {
   return SplitShape{__builtin_ctz(rows_per_block(D)) - a.group_shift, __builtin_ctz(KEYS)};
 }
 
+__device__ __forceinline__ int64_t read_lane(int64_t v, int lane) {
+  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<int32_t>(v), lane);
+  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<int32_t>(v >> 32), lane);
+  return static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
 __device__ __forceinline__ BatchPlan plan_batch(const CtxArgs& a, const SplitShape& sh, int lane) {
   BatchPlan b;
   const bool in = lane < a.n_segments;
   const int s = in ? lane : 0;
   const int64_t q0 = load_index(a.qo_indptr, a.indptr_i64, s), q1 = load_index(a.qo_indptr, a.indptr_i64, s + 1);
   const int64_t k0 = load_index(a.kv_indptr, a.indptr_i64, s), k1 = load_index(a.kv_indptr, a.indptr_i64, s + 1);
-  b.q0 = static_cast<int32_t>(q0);
-  b.k0 = static_cast<int32_t>(k0);
+  b.q0 = q0;
+  b.k0 = k0;
   b.q = in ? static_cast<int32_t>(q1 - q0) : 0;
   b.p = in && a.kv_indices ? static_cast<int32_t>(k1 - k0) : 0;
-  const int32_t cost = segment_cost(sh, b.q, b.p);
-  int32_t sum = cost;
+  const int64_t cost = segment_cost(sh, b.q, b.p);
+  int64_t sum = cost;
 #pragma nounroll
   for (int off = 1; off < a.n_segments; off <<= 1) {
-    const int32_t up = __shfl_up(sum, off);
+    const int64_t up = __shfl_up(sum, off);
     if (lane >= off) sum += up;
   }
   b.before = sum - cost;
-  b.total = __builtin_amdgcn_readlane(sum, a.n_segments - 1);
+  b.total = read_lane(sum, a.n_segments - 1);
   b.live = __builtin_amdgcn_ballot_w64(cost > 0);
   return b;
 }
 
 // Boundary r of this lane (the lanes' searches run side by side).
 __device__ __forceinline__ Place lane_place(const BatchPlan& b, const SplitShape& sh, int32_t heads, int k, int r) {
-  auto get = [&](int i, int32_t* q, int32_t* p, int32_t* before) {
+  auto get = [&](int i, int32_t* q, int32_t* p, int64_t* before) {
     *q = __builtin_amdgcn_readlane(b.q, i);
     *p = __builtin_amdgcn_readlane(b.p, i);
-    *before = __builtin_amdgcn_readlane(b.before, i);
+    *before = read_lane(b.before, i);
   };
   return place_of(sh, get, b.live, b.total, heads, k, r);
 }
 
 __device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+
+__device__ __forceinline__ int64_t uniform(int64_t v) {
+  const uint32_t lo = uniform(static_cast<int32_t>(v)), hi = uniform(static_cast<int32_t>(v >> 32));
+  return static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo);
+}
 
 __device__ __forceinline__ Place uniform(const Place& p) {
   return Place{uniform(p.head), uniform(p.seg), uniform(p.block), uniform(p.tile)};
@@ -309,7 +320,8 @@ constexpr int64_t partial_floats() { return kPartialO + 2 * rows_per_block(D); }
 // query and query count.  The workspace ends with one for every workgroup.
 struct __attribute__((aligned(16))) Cut {
   Place at;
-  int32_t q0, q, pad[2];
+  int64_t q0;
+  int32_t q, pad;
 };
 
 template <int D>
@@ -331,37 +343,6 @@ struct Lds {
   int32_t (&restart)[kRestartWords];  // tile_loop.h
   float2* merge;  // 4 x 16 SUB, split launch only
 };
-
-struct SplitState {
-  Place cur, first, end;
-  uint64_t live;  // segments with queries
-  int32_t rank;
-  int32_t last;  // the part left for last is the one being done
-};
-
-// The next block, segment or head after s.cur in its stretch, then the part
-// left for last; false when the stretch is done.  qlen: s.cur's segment.
-__device__ __forceinline__ bool next_piece(const CtxArgs& a, SplitState& s, int32_t qlen) {
-  if (s.last) return false;
-  bool done = same_block(s.cur, s.end);
-  if (!done) {
-    s.cur.tile = 0;
-    if ((s.cur.block + 1) * a.tokens_per_block < qlen) {
-      ++s.cur.block;
-    } else {
-      s.cur.block = 0;
-      const uint64_t later = s.cur.seg < 63 ? s.live >> (s.cur.seg + 1) << (s.cur.seg + 1) : 0;
-      if (!later) ++s.cur.head;
-      s.cur.seg = __builtin_ctzll(later ? later : s.live);
-    }
-    done = s.cur.head >= a.kv_heads || (same_block(s.cur, s.end) && s.end.tile == 0);
-  }
-  if (!done) return true;
-  if (s.first.tile == 0 || same_block(s.first, s.end)) return false;
-  s.cur = s.first;
-  s.last = 1;
-  return true;
-}
 
 // KEYS keys per tile: 128 for full layers at head_dim 64 (half the tile
 // barriers, staging and commits per key), 64 for windowed layers (less of a
@@ -925,7 +906,7 @@ __global__ void __launch_bounds__(kThreads, 2) context_split_kernel(const CtxArg
   __shared__ int32_t restart[kRestartWords];
   __shared__ float2 merge[4 * 16 * sub_tiles(D)];
   __shared__ SplitState state;
-  __shared__ int4 segments[kMaxSplitSegments];  // first query and prefix index, queries, prefix keys
+  __shared__ Segment segments[kMaxSplitSegments];
   const Lds<D, KEYS, sub_tiles(D)> lds{tile0, tile1, rel_rows, restart, merge};
   {
     const SplitShape shape = split_shape<D, KEYS>(args);
@@ -948,12 +929,12 @@ __global__ void __launch_bounds__(kThreads, 2) context_split_kernel(const CtxArg
     s.last = 0;
     const int32_t qlen = __builtin_amdgcn_readlane(plan.q, s.first.seg);
     if (threadIdx.x == 0)
-      split_cuts<D>(args)[s.rank] = Cut{s.first, __builtin_amdgcn_readlane(plan.q0, s.first.seg), qlen, {0, 0}};
+      split_cuts<D>(args)[s.rank] = Cut{s.first, read_lane(plan.q0, s.first.seg), qlen, 0};
     if (same_block(s.first, s.end) ? s.first.tile == s.end.tile
-                                   : s.first.tile > 0 && !next_piece(args, s, qlen))
+                                   : s.first.tile > 0 && !next_piece(shape, args.kv_heads, s, qlen))
       return;
     if (threadIdx.x == 0) state = s;
-    if (threadIdx.x < kMaxSplitSegments) segments[threadIdx.x] = int4{plan.q0, plan.k0, plan.q, plan.p};
+    if (threadIdx.x < kMaxSplitSegments) segments[threadIdx.x] = Segment{plan.q0, plan.k0, plan.q, plan.p};
     __syncthreads();
   }
   kernel_args* kp = (kernel_args*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -966,8 +947,8 @@ __global__ void __launch_bounds__(kThreads, 2) context_split_kernel(const CtxArg
       // part 2 rank: the stretch's first block, entered past its first tile;
       // part 2 rank + 1: its last, left before its last tile
       float* part = a.partial + (2 * rank + (at.tile > 0 ? 0 : 1)) * partial_floats<D>();
-      const int4 v = segments[at.seg];
-      const Segment sg{uniform(v.x), uniform(v.y), uniform(v.z), uniform(v.w)};
+      const Segment v = segments[at.seg];
+      const Segment sg{uniform(v.q0), uniform(v.k0), uniform(v.q), uniform(v.p)};
       attend<D, KEYS, sub_tiles(D), IdxT, int64_t, false, GEN, true>(a, lds, sg, at.head, at.block, at.tile,
                                                                      same_block(at, end) ? end.tile : -1, part);
     }
@@ -975,10 +956,9 @@ __global__ void __launch_bounds__(kThreads, 2) context_split_kernel(const CtxArg
     s.cur = uniform(s.cur);
     s.first = uniform(s.first);
     s.end = uniform(s.end);
-    s.live = (static_cast<uint64_t>(static_cast<uint32_t>(uniform(static_cast<int32_t>(s.live >> 32)))) << 32) |
-             static_cast<uint32_t>(uniform(static_cast<int32_t>(s.live)));
+    s.live = static_cast<uint64_t>(uniform(static_cast<int64_t>(s.live)));
     s.last = uniform(s.last);
-    if (!next_piece(a, s, uniform(segments[s.cur.seg].z))) return;
+    if (!next_piece(split_shape<D, KEYS>(a), a.kv_heads, s, uniform(segments[s.cur.seg].q))) return;
     __syncthreads();
     if (threadIdx.x == 0) state = s;
     __syncthreads();
@@ -998,7 +978,7 @@ __global__ void __launch_bounds__(512) context_combine_kernel(const CtxArgs a) {
   constexpr int kAhead = 4;  // parts in flight together (8 and 12: most blocks have fewer, 1-6% slower)
   static_assert(64 * kSub * (D / 16 / kCombineDims) == 512, "one wave per row subtile and pair of dim tiles");
   const int lane = threadIdx.x & 63;
-  const int w = uniform(threadIdx.x >> 6);
+  const int w = uniform(static_cast<int32_t>(threadIdx.x >> 6));
   const int s = w % kSub, dt0 = w / kSub * kCombineDims;
   const int wave = blockIdx.x;
   const int r0 = blockIdx.y + 1;
@@ -1013,7 +993,7 @@ __global__ void __launch_bounds__(512) context_combine_kernel(const CtxArgs a) {
   const Place at = from_lane(mine.at, 1), prev = from_lane(mine.at, 0);
   // nothing, or a boundary between two blocks, or not the block's first
   if (at.tile <= 0 || (prev.tile > 0 && same_block(prev, at))) return;
-  const int64_t qo0 = __builtin_amdgcn_readlane(mine.q0, 1);
+  const int64_t qo0 = read_lane(mine.q0, 1);
   const int32_t qlen = __builtin_amdgcn_readlane(mine.q, 1);
   const int32_t t0 = at.block * a.tokens_per_block;
   if (t0 + ((wave * 16 * kSub) >> a.group_shift) >= qlen) return;  // no rows here (nor a part with them)
@@ -1326,10 +1306,7 @@ extern "C" int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t
       q_heads / kv_heads > 128 || head_dim <= 0 || head_dim > 128 || total_queries <= 0 || max_query_len <= 0)
     return 0;
   const int64_t tokens = rows_per_block(head_dim > 64 ? 128 : 64) >> group_shift_of(q_heads / kv_heads);
-  const SplitShape shape{__builtin_ctz(static_cast<uint32_t>(tokens)), head_dim > 64 ? 6 : 7};
-  if (total_prefix < 0 || total_queries > (1 << 30) || total_prefix > (1 << 30) ||
-      cost_bound(shape, n_segments, total_queries, total_prefix) > (1 << 30))
-    return 0;
+  if (total_prefix < 0) return 0;
   const int64_t queries = n_segments == 1 && max_query_len < total_queries ? max_query_len : total_queries;
   // one segment's blocks are known; of several, each leaves half a block empty
   const int64_t blocks = n_segments == 1 ? (queries + tokens - 1) / tokens : queries / tokens + (n_segments + 1) / 2;
