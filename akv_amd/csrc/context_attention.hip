@@ -1142,7 +1142,7 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                                      int32_t positions_dtype, int32_t sliding_window, const float* sinks,
                                      float scale, float logit_cap, void* out, int32_t out_dtype,
                                      int64_t out_stride_t, int64_t out_stride_h, int64_t max_query_len,
-                                     void* workspace, int64_t workspace_bytes, void* stream) {
+                                     bool split, void* workspace, int64_t workspace_bytes, void* stream) {
   if (n_segments < 0 || max_query_len < 0) return fail(AKV_EINVAL, "akv_context_attention: negative size");
   if (n_segments == 0 || max_query_len == 0) return AKV_OK;
   // heads of up to 128 dims in 16-byte chunks: the kernel's 64- or 128-dim
@@ -1162,6 +1162,10 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
     return fail(AKV_EINVAL, "akv_context_attention: index vectors must be int32 or int64");
   if (out_dtype != AKV_BF16 && out_dtype != AKV_F32)
     return fail(AKV_EINVAL, "akv_context_attention: output must be bf16 or f32");
+  if (split && (sliding_window > 0 || n_segments > kMaxSplitSegments || !workspace ||
+                workspace_bytes < split_bytes(head_dim) || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0))
+    return fail(AKV_EINVAL, "akv_context_attention_split: needs no window, at most %d segments and %lld aligned bytes",
+                kMaxSplitSegments, static_cast<long long>(split_bytes(head_dim)));
   if (!q || !k_ext || !v_ext || !out || !qo_indptr || !kv_indptr)
     return fail(AKV_EINVAL, "akv_context_attention: null device pointer");
   // prefix keys are read from the pools through kv_indices
@@ -1227,11 +1231,6 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
   const int64_t blocks = (max_query_len + a.tokens_per_block - 1) / a.tokens_per_block;
   if (blocks * kv_heads > 0x7fffffffLL) return fail(AKV_EINVAL, "akv_context_attention: queries too long");
   a.kv_heads = kv_heads;
-  const bool split = workspace != nullptr;
-  if (split && (a.window >= 0 || n_segments > kMaxSplitSegments || workspace_bytes < split_bytes(head_dim) ||
-                (reinterpret_cast<uintptr_t>(workspace) & 15) != 0))
-    return fail(AKV_EINVAL, "akv_context_attention_split: needs no window, at most %d segments and %lld aligned bytes",
-                kMaxSplitSegments, static_cast<long long>(split_bytes(head_dim)));
   a.n_segments = n_segments;
   a.max_shift = kSplitShift;
   a.partial = static_cast<float*>(workspace);
@@ -1262,7 +1261,7 @@ extern "C" int akv_context_attention(
       v_buffer, k_stride_slot, k_stride_head, v_stride_slot, v_stride_head, n_segments, q_heads, kv_heads, head_dim,
       qo_indptr, kv_indptr, indptr_dtype, kv_indices, indices_dtype, q_positions, kv_positions, positions_dtype,
       sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len,
-      nullptr, 0, stream);
+      false, nullptr, 0, stream);
 }
 
 extern "C" int akv_context_attention_split(
@@ -1280,7 +1279,7 @@ extern "C" int akv_context_attention_split(
       v_buffer, k_stride_slot, k_stride_head, v_stride_slot, v_stride_head, n_segments, q_heads, kv_heads, head_dim,
       qo_indptr, kv_indptr, indptr_dtype, kv_indices, indices_dtype, q_positions, kv_positions, positions_dtype,
       sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len,
-      workspace, workspace_bytes, stream);
+      true, workspace, workspace_bytes, stream);
 }
 
 // Which launch: both times estimated in 64-key tiles of a full block (2.0 us,

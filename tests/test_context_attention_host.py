@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 import torch
 
-from akv_amd import context_attention as ca
+from akv_amd import _lib, context_attention as ca
 
 from harness import attention_metadata, plain_segments, window_segments
 
@@ -29,6 +29,35 @@ def test_validation_messages():
                                 context_kv_positions=torch.zeros(2, dtype=torch.int64))
     with pytest.raises(ValueError, match="custom mask"):
         ca.extend_attention_fwd(q, k, k, q, k, k, ind, ind, ind, torch.ones(1), True, None, 4)
+
+
+def test_split_bytes_names_the_batches_it_takes():
+    need = _lib.load().akv_context_attention_split_bytes
+    assert need(1, 64, 8, 64, -1, 200, 200, 20000) > 0
+    assert need(1, 64, 8, 64, 0, 200, 200, 20000) > 0  # no window either
+    assert need(1, 64, 8, 64, 128, 200, 200, 20000) == 0  # a window
+    assert need(65, 64, 8, 64, -1, 6500, 100, 20000) == 0  # too many segments
+    assert need(1, 64, 8, 64, -1, 4096, 4096, 20000) == 0  # the plain launch fills the chip
+
+
+@pytest.mark.parametrize("why,changes", [("window", {27: 128}), ("segments", {15: 65}), ("no workspace", {36: None}),
+                                         ("short workspace", {37: 64}), ("workspace alignment", {36: (1 << 20) + 8})])
+def test_split_refuses(why, changes):
+    """Each is refused before any device pointer is looked at: all of them
+    are null here, so a call that passed this check would stop at the next."""
+    lib = _lib.load()
+    fn = lib.akv_context_attention_split
+    args = [None if t is _lib.c_void_p else 0 for t in fn.argtypes]
+    good = {15: 1, 16: 8, 17: 1, 18: 64, 21: _lib.AKV_I32, 23: _lib.AKV_I32, 26: _lib.AKV_I32, 27: -1, 29: 0.125,
+            32: _lib.AKV_BF16, 35: 4, 36: 1 << 20, 37: 1 << 30}
+    for at, value in {**good, **changes}.items():
+        args[at] = value
+    assert fn(*args) == _lib.AKV_EINVAL
+    assert "akv_context_attention_split: needs no window" in _lib.last_error(), why
+    for at, value in good.items():
+        args[at] = value
+    assert fn(*args) == _lib.AKV_EINVAL
+    assert "null device pointer" in _lib.last_error()
 
 
 def test_metadata_helper_splits_segments():

@@ -119,18 +119,3 @@ def test_windows_at_the_block_size_rule(device, window, positions):
     c = _case(device, 16, 2, 64, [300, 17], [900, 40], seed=window)
     got, want = _run(device, c, window=window, positions=positions, sinks=None, out_dtype=torch.float32, scale=0.125)
     assert np.abs(got - want).max() <= TOL
-
-
-def test_split_rejects_a_window_and_a_short_workspace():
-    lib = _lib.load()
-    assert lib.akv_context_attention_split_bytes(1, 64, 8, 64, 128, 200, 200, 20000) == 0
-    assert lib.akv_context_attention_split_bytes(65, 64, 8, 64, -1, 6500, 100, 20000) == 0
-    assert lib.akv_context_attention_split_bytes(1, 64, 8, 64, -1, 4096, 4096, 20000) == 0
-    fn = lib.akv_context_attention_split
-    args = [None if t is _lib.c_void_p else 0 for t in fn.argtypes]
-    fake = 1 << 20
-    for i, v in {0: fake, 3: fake, 4: fake, 15: 1, 16: 8, 17: 1, 18: 64, 19: fake, 20: fake, 29: 0.125, 31: fake,
-                 35: 4, 36: fake, 37: 64}.items():
-        args[i] = v
-    assert fn(*args) == _lib.AKV_EINVAL
-    assert "aligned bytes" in _lib.last_error()
