@@ -23,8 +23,8 @@
 //
 // MFMA 16x16x32 bf16 lane layout (verified on gfx950): lane l supplies
 // A[l%16][k(l, i)] and B[k(l, i)][l%16], i < 8, and holds D[4(l/16)+i][l%16].
+#include <algorithm>
 #include <cmath>
-
 #include <mutex>
 
 #include "common.h"
@@ -60,10 +60,34 @@ struct AttnArgs {
   int32_t out_f32;
   int64_t out_stride_b, out_stride_h;
   int32_t n_requests, q_heads, kv_heads, group, chunks;
-  int32_t chunk_keys;  // keys per workgroup, a multiple of kPass
+  int32_t max_passes;  // passes per workgroup with which `chunks` chunks hold max_len keys
+  // the grid: chunks fastest, then heads or requests; its chunks turn by one
+  // every 2^turn_shift (request, head) pairs, and again every 4 and 32 times that
+  int32_t heads_last, turn_shift;
   int32_t q_vectors;   // q rows are 16-byte aligned
   float* partial;  // [B][Hkv][chunks][16][D + 2]  (o..., m, l)
 };
+
+// Passes of a workgroup: up to four where that still leaves eight workgroups
+// per CU (a quarter of the partial results).
+constexpr int32_t kMaxPasses = 4;
+constexpr int64_t kEnoughGroups = 8 * 256;
+
+// Keys of a chunk of a request of `len` keys in a batch of `total`.  The host
+// knows a bound of the longest request only, which may be far off (a captured
+// graph's, a context length); the batch itself says how many workgroups its
+// keys can feed.  Both kernels compute it.
+__device__ __forceinline__ int32_t chunk_keys_of(const AttnArgs& a, int32_t len, int32_t total) {
+  int32_t passes = 1;
+  while (passes < a.max_passes && (static_cast<int64_t>(total) * a.kv_heads >= kEnoughGroups * 2 * passes * kPass ||
+                                   len > static_cast<int64_t>(a.chunks) * passes * kPass))
+    passes *= 2;
+  // one chunk of two passes rather than two of one
+  if (passes == 1 && a.max_passes > 1 && len <= 2 * kPass) passes = 2;
+  // equal chunks, in whole waves of keys
+  const uint32_t most = passes * kPass, n = (static_cast<uint32_t>(len) + most - 1) / most;
+  return n > 1 ? ((static_cast<uint32_t>(len) + n - 1) / n + 63) / 64 * 64 : most;
+}
 
 // The V rows of keys past a chunk's end: their weights are 0, and 0 times
 // whatever a real row holds (infinities) need not be 0.
@@ -74,13 +98,27 @@ static __device__ __attribute__((aligned(16))) const uint32_t zero_row[64] = {};
 template <int D>
 __device__ __forceinline__ int swz(int r) { return D == 64 ? r & 6 : (r & 7) << 1; }
 
-// Bound by the HBM's random rows: 32 GPT-OSS requests of ~20k keys (1.29 GB)
-// take 247 us, 5.2 TB/s, where a large copy reaches 4.9 (read + write); with one
-// wave per 256 keys, 16 at a time, they took 256.  Four requests of 1-6k keys,
-// where the chain of round trips counts, take 10 us against 20; a 128-key
-// window 6-7 us against 12-13.  Grid: chunks fastest, so neighbouring
-// workgroups read different rows; a chunk's KV heads one after the other on
-// one XCD measured 4% slower (295 against 284 us for the decode step).
+// Bound by the HBM's random rows: 32 GPT-OSS requests of ~20k keys (1.31 GB)
+// take 252 us with the combine, 5.2 TB/s, where a large copy reaches 4.9 (read
+// + write); with one wave per 256 keys, 16 at a time, they took 267.  Four
+// requests of 1-6k keys, where the chain of round trips counts, take 12 us
+// against 22; a 128-key window 4.3 against 9.3.  The next pass's slots arrive
+// with this pass's rows (12 Llama-3 requests and the like 2-8%).
+//
+// The grid follows the host's bound, so its live workgroups must not depend
+// on where they stand in it: workgroups go round robin to the XCDs, and within
+// an XCD to its shader engines, so a grid whose first chunks are the live (or
+// the long) ones would keep to a few of them.  Its chunks therefore turn from
+// pair to pair, at the period of the XCDs and at 4 and 32 times that, and a
+// request's chunks are equally long.  Without both, and with passes from the
+// bound: 64 GPT-OSS requests of 2000 keys at a bound of 32768 took 372 us (52
+// now), 300 of 1100 at 1100 232 (156), 128 of 100-8000 218 (133).  Chunks
+// fastest and then heads, so neighbouring workgroups read different rows;
+// where there are few chunks (kFewChunks), requests before heads: 256 x 1000
+// keys of all heads side by side 4.4 TB/s, of different requests 5.5; with 20
+// chunks it is 0.4-1% slower, and 5% for ragged requests.  A chunk's heads one
+// after the other on one XCD measured 4% slower (295 against 284 us for the
+// decode step).
 template <int D>
 __global__ void __launch_bounds__(4 * D, 4) decode_attention_partial_kernel(const AttnArgs a) {
   constexpr int kWaves = D / 16;
@@ -97,15 +135,22 @@ __global__ void __launch_bounds__(4 * D, 4) decode_attention_partial_kernel(cons
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int chunk = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+  const int b = a.heads_last ? blockIdx.y : blockIdx.z;
+  const int g = a.heads_last ? blockIdx.z : blockIdx.y;
+  const uint32_t pair = (blockIdx.z * gridDim.y + blockIdx.y) >> a.turn_shift;
+  const uint32_t turn = pair + (pair >> 2) + (pair >> 5);
+  int chunk = blockIdx.x + turn % a.chunks;
+  if (chunk >= a.chunks) chunk -= a.chunks;
   const int64_t begin = a.kv_indptr[b];
-  const int64_t len = a.kv_indptr[b + 1] - begin;
+  const int32_t len = max(a.kv_indptr[b + 1] - a.kv_indptr[b], 0);
+  const int32_t total = a.kv_indptr[a.n_requests] - a.kv_indptr[0];
   // a closed gate stops the workgroup before its key indices and rows
   if (gated(a.gate)) return;
-  const int64_t c0 = static_cast<int64_t>(chunk) * a.chunk_keys;
+  const int32_t chunk_keys = chunk_keys_of(a, len, total);
+  const int64_t c0 = static_cast<int64_t>(chunk) * chunk_keys;
   // an empty chunk is not read by the combine; with one chunk the output is 0
   if (c0 >= len && a.chunks > 1) return;
-  const int n = static_cast<int>(len - c0 < a.chunk_keys ? (len > c0 ? len - c0 : 0) : a.chunk_keys);
+  const int n = static_cast<int>(len - c0 < chunk_keys ? (len > c0 ? len - c0 : 0) : chunk_keys);
   const int32_t* idx = a.kv_indices + begin + c0;
   const int col = lane & 15;   // head within the group (B / D layout column)
   const int quad = lane >> 4;  // 0..3
@@ -136,10 +181,14 @@ __global__ void __launch_bounds__(4 * D, 4) decode_attention_partial_kernel(cons
   float m_run = -INFINITY, l_run = 0.f;
   __bf16* vt = reinterpret_cast<__bf16*>(tiles[wave]);
 
-  for (int t0 = wave * kKeys; t0 < n; t0 += kPass) {
-    // this lane's key of the pass (keys past the end: the last one's row)
+  // the slot of this lane's key of a pass (keys past the end: the last one's)
+  auto slot_at = [&](int t0) {
     const int mine = t0 + (lane & (kKeys - 1));
-    const int32_t slot = idx[mine < n ? mine : n - 1];
+    return idx[mine < n ? mine : n - 1];
+  };
+  int32_t next = wave * kKeys < n ? slot_at(wave * kKeys) : 0;
+  for (int t0 = wave * kKeys; t0 < n; t0 += kPass) {
+    const int32_t slot = next;
     u32x4 k[kTiles][kSteps];
 #pragma unroll
     for (int j = 0; j < kTiles; ++j) {
@@ -155,6 +204,8 @@ __global__ void __launch_bounds__(4 * D, 4) decode_attention_partial_kernel(cons
       if (t0 + r >= n) row = reinterpret_cast<const char*>(zero_row);
       __builtin_amdgcn_global_load_lds(row + 16 * c, (lds_void*)(vt + u * kRows * D), 16, 0, 0);
     }
+    // the next pass's slots come in with these rows
+    if (t0 + kPass < n) next = slot_at(t0 + kPass);
     // ---- S^T = K . Q^T; lane holds S^T[keys 16 j + 4 quad + i][head col]
     f32x4 p[kTiles];
     float top = -INFINITY;
@@ -284,11 +335,13 @@ __global__ void __launch_bounds__(kCombineThreads) decode_attention_combine_kern
   const int hl = h - g * a.group;
   const int dl = threadIdx.x % kLanes;
   const int way = threadIdx.x / kLanes;
-  const int64_t len = a.kv_indptr[b + 1] - a.kv_indptr[b];
+  const int32_t len = max(a.kv_indptr[b + 1] - a.kv_indptr[b], 0);
+  const int32_t total = a.kv_indptr[a.n_requests] - a.kv_indptr[0];
   if (gated(a.gate)) return;
   // keys past max_len (a caller error) are not read: the partials stop there
-  const int64_t want = (len + a.chunk_keys - 1) / a.chunk_keys;
-  const int used = static_cast<int>(want < a.chunks ? want : a.chunks);
+  const uint32_t chunk_keys = chunk_keys_of(a, len, total);
+  const int want = (static_cast<uint32_t>(len) + chunk_keys - 1) / chunk_keys;
+  const int used = want < a.chunks ? want : a.chunks;
   const float* base = a.partial + (static_cast<int64_t>(b) * a.kv_heads + g) * a.chunks * 16 * (D + 2);
   float m = -INFINITY, l = 0.f;
   f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -340,19 +393,18 @@ __global__ void __launch_bounds__(kCombineThreads) decode_attention_combine_kern
 
 int64_t chunks_for(int64_t max_len, int64_t keys) { return max_len <= 0 ? 1 : (max_len + keys - 1) / keys; }
 
-// Passes of a workgroup: up to four where that still leaves eight workgroups
-// per CU (a quarter of the partial results), and two keys' worth of passes
-// rather than a second launch for requests that then fit one chunk.
-constexpr int kMaxPasses = 4;
-constexpr int64_t kEnoughGroups = 8 * 256;
-int32_t chunk_keys_for(int64_t requests, int64_t kv_heads, int64_t max_len) {
+// The passes that the bound allows, and two for requests of up to two passes'
+// keys rather than a second launch.
+int32_t max_passes_for(int64_t requests, int64_t kv_heads, int64_t max_len) {
   int32_t passes = 1;
   while (passes < kMaxPasses &&
          requests * kv_heads * chunks_for(max_len, 2 * passes * kPass) >= kEnoughGroups)
     passes *= 2;
   if (passes == 1 && max_len <= 2 * kPass) passes = 2;
-  return passes * kPass;
+  return passes;
 }
+
+constexpr int32_t kFewChunks = 8;
 
 // Split-K scratch of akv_decode_attention_noalloc: a file-scope device array,
 // one per GPU, held until the process ends.  Host code never passes the
@@ -449,13 +501,16 @@ extern "C" int akv_decode_attention(const void* q, int64_t q_stride_b, int64_t q
   a.q_heads = q_heads;
   a.kv_heads = kv_heads;
   a.group = q_heads / kv_heads;
-  a.chunk_keys = chunk_keys_for(n_requests, kv_heads, max_len);
-  a.chunks = static_cast<int32_t>(chunks_for(max_len, a.chunk_keys));
+  a.max_passes = max_passes_for(n_requests, kv_heads, max_len);
+  a.chunks = static_cast<int32_t>(chunks_for(max_len, a.max_passes * kPass));
+  a.heads_last = a.chunks < kFewChunks;
+  // 2^e chunks (times an odd number) of 2^(3-e) pairs are one round of the XCDs
+  a.turn_shift = 3 - std::min(3, __builtin_ctz(static_cast<uint32_t>(a.chunks)));
   a.q_vectors = ((q_stride_b | q_stride_h) % 8 == 0) && (reinterpret_cast<uintptr_t>(q) & 15) == 0;
   a.partial = static_cast<float*>(workspace);
   hipStream_t st = as_stream(stream);
-  const dim3 grid(static_cast<unsigned>(a.chunks), static_cast<unsigned>(kv_heads),
-                  static_cast<unsigned>(n_requests));
+  const unsigned heads = static_cast<unsigned>(kv_heads), requests = static_cast<unsigned>(n_requests);
+  const dim3 grid(static_cast<unsigned>(a.chunks), a.heads_last ? requests : heads, a.heads_last ? heads : requests);
   if (head_dim == 64)
     hipLaunchKernelGGL(decode_attention_partial_kernel<64>, grid, dim3(256), 0, st, a);
   else
