@@ -88,6 +88,12 @@ _SIGNATURES = {
          c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, _P, _P, c_int32, _P, c_int32, _P, _P,
          c_int32, c_int32, _P, ctypes.c_float, ctypes.c_float, _P, c_int32, c_int64, c_int64, c_int64, _P],
     ),
+    "akv_context_attention_sized": (
+        c_int32,
+        [_P, c_int64, c_int64, _P, _P, c_int64, c_int64, c_int64, c_int64, _P, _P, c_int64, c_int64,
+         c_int64, c_int64, c_int32, c_int32, c_int32, c_int32, _P, _P, c_int32, _P, c_int32, _P, _P,
+         c_int32, c_int32, _P, ctypes.c_float, ctypes.c_float, _P, c_int32, c_int64, c_int64, c_int64, c_int64, _P],
+    ),
     "akv_context_attention_split": (
         c_int32,
         [_P, c_int64, c_int64, _P, _P, c_int64, c_int64, c_int64, c_int64, _P, _P, c_int64, c_int64,

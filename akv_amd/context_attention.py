@@ -5,7 +5,7 @@ context positions (``akv/system/sglang.patch:106-237``): same arguments,
 checks and messages.  The reference's prefill metadata builder
 (``context_backend.py:24-251``) passes it qo/kv indptrs, the bound prefix
 slots and the query / key positions unchanged.  The device work is
-``akv_context_attention`` in ``libakv_amd.so``; there is no other path.
+``akv_context_attention_sized`` (or ``_split``) in ``libakv_amd.so``; there is no other path.
 """
 
 from __future__ import annotations
@@ -102,7 +102,7 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
                                      kv_indices.numel())
         stream = current_stream_handle(q_extend.device)
         if workspace is None:
-            rc = lib.akv_context_attention(*args, stream)
+            rc = lib.akv_context_attention_sized(*args, q_extend.shape[0], stream)
         else:
             rc = lib.akv_context_attention_split(*args, workspace.data_ptr(), workspace.numel(), stream)
     _lib.check(rc, "akv_context_attention")

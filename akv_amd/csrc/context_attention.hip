@@ -91,10 +91,8 @@ constexpr int kWaves = 8;
 // (token, head) rows of a block with `sub` row subtiles per wave
 constexpr int block_rows(int sub) { return kWaves * 16 * sub; }
 constexpr int rows_per_block(int d) { return block_rows(sub_tiles(d)); }
-// Windows up to kNarrowWindow at head_dim 64 take blocks of kNarrowSub subtiles per wave.  A
-// block of few tokens sees few keys outside its rows' windows, and its tiles
-// are short, where a 128-key window's cost is mostly one tile's latency after
-// another; wide windows share each tile over as many rows as full layers do.
+// Blocks of a narrow window (up to kNarrowWindow, 64-dim tiles) may have
+// kNarrowSub subtiles per wave (narrow_blocks).
 constexpr int kNarrowWindow = 512;
 constexpr int kNarrowSub = 1;
 constexpr int kThreads = 64 * kWaves;
@@ -1101,13 +1099,44 @@ void launch_idx(bool idx64, int pos, dim3 grid, hipStream_t st, const CtxArgs& a
     launch_gen<D, KEYS, SUB, int32_t>(pos, grid, st, a);
 }
 
-void launch_typed(bool split, bool idx64, int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
+// Whether a window takes blocks of a quarter of the rows.  Such a block sees
+// few keys outside its rows' windows, and two of them share a CU, which hides
+// the latency that a narrow window's few tiles consist of; but there are four
+// times as many, and each stages its own window.  Full blocks run in whole
+// rounds of 256, counted with the empty ones of a ragged batch's grid (the
+// CUs that meet those wait all the same); short ones, 512 at once, even out.
+// Times in microseconds, fitted to full | short blocks of one segment with
+// GPT-OSS heads at windows 64, 128, 256, 512:
+//   1000 tokens (half a round):  18.6 | 11.3, 20.6 | 13.5, 24.4 | 16.4, 32.2 | 22.0
+//   2000 (one):                  21.5 | 20.6, 23.4 | 23.3, 27.1 | 29.0, 35.2 | 39.3
+//   3000 (one and a half):       39.5 | 30.6, 43.0 | 33.8, 50.8 | 41.7, 66.2 | 57.0
+//   8192 (four):                 80.1 | 68.9, 87.7 | 76.7, 103.7 | 94.5, 134.3 | 133.8
+// Heads of 32 dims (full blocks load less, short ones still clear their tiles)
+// at window 128: 2000 tokens 18.2 | 22.2, 3000 34.2 | 31.5.  512-token blocks
+// (group 1), 4096 tokens: 54.7 | 30.8.  Six segments of 33-600 tokens, window
+// 128 and 512: 38.4 | 24.0, 63.5 | 40.3.
+bool narrow_blocks(int32_t head_dim, int32_t group_shift, int32_t window, int64_t kv_heads, int64_t segments,
+                   int64_t max_query_len, int64_t total_queries) {
+  if (head_dim > 64 || window < 0 || window > kNarrowWindow) return false;
+  const int64_t full = block_rows(sub_tiles(64)) >> group_shift, part = block_rows(kNarrowSub) >> group_shift;
+  const int64_t full_blocks = (max_query_len + full - 1) / full * segments;
+  int64_t part_blocks = (max_query_len + part - 1) / part * segments;
+  // of unequal segments, each leaves half a block empty
+  if (total_queries > 0 && total_queries < max_query_len * segments)
+    part_blocks = std::min(part_blocks, total_queries / part + (segments + 1) / 2);
+  const double full_round = 9. + 11. * head_dim / 64. + 0.027 * window + 0.085 * std::max<int64_t>(0, full - 64);
+  const double part_round = 6.3 + 0.02 * window + 0.028 * part;
+  return 1.02 * (6. + part_round * std::max(1., part_blocks * kv_heads / 512.)) <
+         full_round * ((full_blocks * kv_heads + 255) / 256);
+}
+
+void launch_typed(bool split, bool narrow, bool idx64, int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
   const bool wide = a.head_dim > 64;
   if (split)
     wide ? launch_idx<128, 64, 0>(idx64, pos, grid, st, a) : launch_idx<64, 128, 0>(idx64, pos, grid, st, a);
   else if (wide)
     launch_idx<128, 64, sub_tiles(128)>(idx64, pos, grid, st, a);
-  else if (a.window >= 0 && a.window <= kNarrowWindow)
+  else if (narrow)
     launch_idx<64, 64, kNarrowSub>(idx64, pos, grid, st, a);
   else if (a.window >= 0)
     launch_idx<64, 64, sub_tiles(64)>(idx64, pos, grid, st, a);
@@ -1142,7 +1171,7 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
                                      int32_t positions_dtype, int32_t sliding_window, const float* sinks,
                                      float scale, float logit_cap, void* out, int32_t out_dtype,
                                      int64_t out_stride_t, int64_t out_stride_h, int64_t max_query_len,
-                                     bool split, void* workspace, int64_t workspace_bytes, void* stream) {
+                                     int64_t total_queries, bool split, void* workspace, int64_t workspace_bytes, void* stream) {
   if (n_segments < 0 || max_query_len < 0) return fail(AKV_EINVAL, "akv_context_attention: negative size");
   if (n_segments == 0 || max_query_len == 0) return AKV_OK;
   // heads of up to 128 dims in 16-byte chunks: the kernel's 64- or 128-dim
@@ -1223,8 +1252,9 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
   a.group = q_heads / kv_heads;
   a.group_shift = group_shift_of(a.group);
   const int tile_dim = head_dim > 64 ? 128 : 64;
-  const int sub = tile_dim == 64 && a.window >= 0 && a.window <= kNarrowWindow ? kNarrowSub : sub_tiles(tile_dim);
-  a.tokens_per_block = block_rows(sub) >> a.group_shift;
+  const bool narrow = narrow_blocks(head_dim, a.group_shift, a.window, kv_heads, n_segments, max_query_len,
+                                    total_queries);
+  a.tokens_per_block = block_rows(narrow ? kNarrowSub : sub_tiles(tile_dim)) >> a.group_shift;
   a.head_dim = head_dim;
   a.cap = logit_cap;
   a.cap_log2 = logit_cap * kLog2e;
@@ -1239,12 +1269,30 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
   hipStream_t st = as_stream(stream);
   const bool idx64 = indices_dtype == AKV_I64;
   const int pos = q_positions == nullptr || a.window < 0 ? 0 : (positions_dtype == AKV_I64 ? 2 : 1);
-  launch_typed(split, idx64, pos, grid, st, a);
+  launch_typed(split, narrow, idx64, pos, grid, st, a);
   return check_launch("akv_context_attention");
 }
 
 }  // namespace
 }  // namespace akv
+
+extern "C" int akv_context_attention_sized(
+    const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_ext,
+    const void* v_ext, int64_t k_ext_stride_t, int64_t k_ext_stride_h, int64_t v_ext_stride_t, int64_t v_ext_stride_h,
+    const void* k_buffer, const void* v_buffer, int64_t k_stride_slot, int64_t k_stride_head, int64_t v_stride_slot,
+    int64_t v_stride_head, int32_t n_segments, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+    const void* qo_indptr, const void* kv_indptr, int32_t indptr_dtype, const void* kv_indices, int32_t indices_dtype,
+    const void* q_positions, const void* kv_positions, int32_t positions_dtype, int32_t sliding_window,
+    const float* sinks, float scale, float logit_cap, void* out, int32_t out_dtype, int64_t out_stride_t,
+    int64_t out_stride_h, int64_t max_query_len, int64_t total_queries,
+    void* stream) {
+  return akv::run_context_attention(
+      q, q_stride_t, q_stride_h, k_ext, v_ext, k_ext_stride_t, k_ext_stride_h, v_ext_stride_t, v_ext_stride_h, k_buffer,
+      v_buffer, k_stride_slot, k_stride_head, v_stride_slot, v_stride_head, n_segments, q_heads, kv_heads, head_dim,
+      qo_indptr, kv_indptr, indptr_dtype, kv_indices, indices_dtype, q_positions, kv_positions, positions_dtype,
+      sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len,
+      total_queries, false, nullptr, 0, stream);
+}
 
 extern "C" int akv_context_attention(
     const void* q, int64_t q_stride_t, int64_t q_stride_h, const void* k_ext,
@@ -1256,12 +1304,11 @@ extern "C" int akv_context_attention(
     const float* sinks, float scale, float logit_cap, void* out, int32_t out_dtype, int64_t out_stride_t,
     int64_t out_stride_h, int64_t max_query_len,
     void* stream) {
-  return akv::run_context_attention(
+  return akv_context_attention_sized(
       q, q_stride_t, q_stride_h, k_ext, v_ext, k_ext_stride_t, k_ext_stride_h, v_ext_stride_t, v_ext_stride_h, k_buffer,
       v_buffer, k_stride_slot, k_stride_head, v_stride_slot, v_stride_head, n_segments, q_heads, kv_heads, head_dim,
       qo_indptr, kv_indptr, indptr_dtype, kv_indices, indices_dtype, q_positions, kv_positions, positions_dtype,
-      sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len,
-      false, nullptr, 0, stream);
+      sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len, 0, stream);
 }
 
 extern "C" int akv_context_attention_split(
@@ -1279,7 +1326,7 @@ extern "C" int akv_context_attention_split(
       v_buffer, k_stride_slot, k_stride_head, v_stride_slot, v_stride_head, n_segments, q_heads, kv_heads, head_dim,
       qo_indptr, kv_indptr, indptr_dtype, kv_indices, indices_dtype, q_positions, kv_positions, positions_dtype,
       sliding_window, sinks, scale, logit_cap, out, out_dtype, out_stride_t, out_stride_h, max_query_len,
-      true, workspace, workspace_bytes, stream);
+      0, true, workspace, workspace_bytes, stream);
 }
 
 // Which launch: both times estimated in 64-key tiles of a full block (2.0 us,

@@ -419,6 +419,31 @@ int akv_context_attention(const void* q, int64_t q_stride_t,
                           void* stream);
 
 /*
+ * The same, with the number of query tokens that the segments hold together
+ * (0: not known), which a ragged batch's max_query_len does not tell: a window
+ * chooses its blocks by it.  The results do not depend on it beyond rounding.
+ */
+int akv_context_attention_sized(const void* q, int64_t q_stride_t,
+                          int64_t q_stride_h, const void* k_ext,
+                          const void* v_ext, int64_t k_ext_stride_t,
+                          int64_t k_ext_stride_h, int64_t v_ext_stride_t,
+                          int64_t v_ext_stride_h, const void* k_buffer,
+                          const void* v_buffer, int64_t k_stride_slot,
+                          int64_t k_stride_head, int64_t v_stride_slot,
+                          int64_t v_stride_head, int32_t n_segments,
+                          int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+                          const void* qo_indptr, const void* kv_indptr,
+                          int32_t indptr_dtype, const void* kv_indices,
+                          int32_t indices_dtype, const void* q_positions,
+                          const void* kv_positions, int32_t positions_dtype,
+                          int32_t sliding_window, const float* sinks,
+                          float scale, float logit_cap, void* out,
+                          int32_t out_dtype, int64_t out_stride_t,
+                          int64_t out_stride_h, int64_t max_query_len,
+                          int64_t total_queries,
+                          void* stream);
+
+/*
  * The same attention with the keys of each block of queries shared out over
  * one workgroup per CU: for batches without a sliding window whose blocks of
  * queries would leave CUs idle.  Partial results of blocks whose keys were

@@ -112,10 +112,30 @@ def test_split_matches_plain(device, monkeypatch, d, idx, ind, pos, segments):
     assert (got - want).abs().max() <= 2e-2
 
 
+# heads, head_dim, queries, prefixes; the last two fill a round of full blocks
+@pytest.mark.parametrize("hq,hkv,d,q_lens,p_lens", [(16, 2, 64, [300, 17], [900, 40]), (32, 1, 64, [65, 9], [700, 20]),
+                                                    (128, 1, 64, [7, 33], [600, 530]), (14, 2, 32, [130, 1], [20, 600]),
+                                                    (64, 8, 64, [64] * 32, [30] * 32), (64, 8, 32, [63] * 32, [70] * 32)])
 @pytest.mark.parametrize("positions", [True, False])
-@pytest.mark.parametrize("window", [1, 511, 512, 513, 700])
-def test_windows_at_the_block_size_rule(device, window, positions):
-    """Windows up to 512 take blocks of few tokens, wider ones full blocks."""
-    c = _case(device, 16, 2, 64, [300, 17], [900, 40], seed=window)
+@pytest.mark.parametrize("window", [1, 256, 511, 512, 513, 700])
+def test_windows_at_the_block_size_rule(device, hq, hkv, d, q_lens, p_lens, window, positions):
+    """Blocks of a quarter of the rows (down to one token) where the window
+    and the batch call for them, full blocks otherwise."""
+    c = _case(device, hq, hkv, d, q_lens, p_lens, seed=window)
     got, want = _run(device, c, window=window, positions=positions, sinks=None, out_dtype=torch.float32, scale=0.125)
+    assert np.abs(got - want).max() <= TOL
+
+
+@pytest.mark.parametrize("window", [-1, 128, 600])
+def test_without_the_queries_count(device, monkeypatch, window):
+    """The entry that is not told how many queries the segments hold."""
+    lib = _lib.load()
+
+    class Unsized:
+        akv_context_attention_split_bytes = staticmethod(lambda *a: 0)
+        akv_context_attention_sized = staticmethod(lambda *a: lib.akv_context_attention(*a[:-2], a[-1]))
+
+    monkeypatch.setattr(ca._lib, "calls", lambda: Unsized)
+    c = _case(device, 16, 2, 64, [300, 17, 90], [900, 40, 300], seed=window + 2)
+    got, want = _run(device, c, window=window, positions=True, sinks=None, out_dtype=torch.bfloat16, scale=0.125)
     assert np.abs(got - want).max() <= TOL
