@@ -1355,13 +1355,22 @@ extern "C" int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t
   if (total_prefix < 0) return 0;
   const int64_t queries = n_segments == 1 && max_query_len < total_queries ? max_query_len : total_queries;
   // one segment's blocks are known; of several, each leaves half a block empty
-  const int64_t blocks = n_segments == 1 ? (queries + tokens - 1) / tokens : queries / tokens + (n_segments + 1) / 2;
+  const int64_t most = (std::min(queries, max_query_len) + tokens - 1) / tokens * n_segments;
+  const int64_t blocks = n_segments == 1 ? most : std::min(most, queries / tokens + (n_segments + 1) / 2);
   const int64_t groups = blocks * kv_heads, rounds = (groups + kSplitGroups - 1) / kSplitGroups;
   const int64_t prefix = total_prefix / n_segments, own = queries / n_segments / 2;
-  const int64_t longest = (n_segments == 1 ? prefix : prefix + prefix / 2) + own;
+  // how unequal several prefixes are is not known: for equal ones that fill
+  // whole rounds the plain launch is the better one (64 segments of 9-28 queries,
+  // 28 / 4 heads x 128, over ~1900 keys: 99 plain, 104 split; 32 of 7-29, 40 / 8
+  // heads, over 2268: 100 | 124)
+  const int64_t longest = (n_segments == 1 ? prefix : prefix + prefix / 4) + own;
   const double share = static_cast<double>(groups) / kSplitGroups, tiles = (prefix + own) / 64.;
   const double plain = 6. + std::min(rounds * (longest / 64.), (share + 1.) * tiles);
-  const double split = 1.06 * share * tiles + 5. * (share + 1.) + 9.;
+  double split = 1.06 * share * tiles + 5. * (share + 1.) + 9.;
+  // more heads than XCDs: an XCD's workgroups walk the keys of several heads
+  // (6 x 682 new tokens, 16 heads x 64 over 1000 keys: 67 plain, 70 split; 64
+  // heads x 128 over 5000: 972 | 1018)
+  if (kv_heads > 8) split *= 1.15;
   if (plain <= split) return 0;
   return split_bytes(head_dim);
 }
