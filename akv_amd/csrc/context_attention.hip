@@ -1366,11 +1366,10 @@ extern "C" int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t
   const int64_t longest = (n_segments == 1 ? prefix : prefix + prefix / 4) + own;
   const double share = static_cast<double>(groups) / kSplitGroups, tiles = (prefix + own) / 64.;
   const double plain = 6. + std::min(rounds * (longest / 64.), (share + 1.) * tiles);
-  double split = 1.06 * share * tiles + 5. * (share + 1.) + 9.;
   // more heads than XCDs: an XCD's workgroups walk the keys of several heads
-  // (6 x 682 new tokens, 16 heads x 64 over 1000 keys: 67 plain, 70 split; 64
-  // heads x 128 over 5000: 972 | 1018)
-  if (kv_heads > 8) split *= 1.15;
+  // (6 x 682 new tokens over 5000 keys, 64 heads x 128: 972 plain, 1018 split)
+  const double tile = kv_heads > 8 ? 1.06 * 1.08 : 1.06;
+  const double split = tile * share * tiles + 5. * (share + 1.) + 9.;
   if (plain <= split) return 0;
   return split_bytes(head_dim);
 }
