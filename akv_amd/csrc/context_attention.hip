@@ -125,7 +125,7 @@ struct CtxArgs {
   float cap, cap_log2;  // logit cap (scores -> cap tanh(score / cap)), cap log2(e)
   // split launch only
   int32_t n_segments;
-  int32_t max_shift;    // log2 of the workgroups
+  int32_t max_shift;    // log2 of the workgroups (what the workspace holds)
   float* partial;       // kPartialFloats per part, two parts per workgroup
 };
 
@@ -199,7 +199,7 @@ __device__ __forceinline__ int32_t rel_pos(int64_t p, int64_t base) {
   return static_cast<int32_t>(r < -kFar ? -kFar : (r > kFar ? kFar : r));
 }
 
-// Workgroups of a split launch: one per CU (a power of two).
+// Most workgroups of a split launch: one per CU (a power of two).
 constexpr int kSplitShift = 8;
 constexpr int kSplitGroups = 1 << kSplitShift;
 // The split launch keeps a batch's segments one to a lane.
@@ -324,7 +324,7 @@ struct __attribute__((aligned(16))) Cut {
 
 template <int D>
 __device__ __forceinline__ Cut* split_cuts(const CtxArgs& a) {
-  return reinterpret_cast<Cut*>(a.partial + 2 * kSplitGroups * partial_floats<D>());
+  return reinterpret_cast<Cut*>(a.partial + (partial_floats<D>() << (a.max_shift + 1)));
 }
 
 // A segment's first query and prefix index, its queries and prefix keys.
@@ -983,8 +983,9 @@ __global__ void __launch_bounds__(512) context_combine_kernel(const CtxArgs a) {
   // lane i: boundary r0 - 1 + i
   const Cut* cuts = split_cuts<D>(a);
   auto load_cut = [&](int r) {
-    Cut c = cuts[r < kSplitGroups ? r : 0];
-    if (r >= kSplitGroups) c.at.tile = -1;
+    const bool in = r < 1 << a.max_shift;
+    Cut c = cuts[in ? r : 0];
+    if (!in) c.at.tile = -1;
     return c;
   };
   Cut mine = load_cut(r0 - 1 + lane);
@@ -1066,7 +1067,8 @@ void launch_pos(int pos, dim3 grid, hipStream_t st, const CtxArgs& a) {
   // neither a split launch nor one of 128-key tiles has one
   if constexpr (SUB == 0) {
     hipLaunchKernelGGL((context_split_kernel<D, KEYS, IdxT, GEN>), grid, dim3(kThreads), 0, st, a);
-    hipLaunchKernelGGL((context_combine_kernel<D, GEN>), dim3(kWaves, grid.x - 1), dim3(512), 0, st, a);
+    if (grid.x > 1)
+      hipLaunchKernelGGL((context_combine_kernel<D, GEN>), dim3(kWaves, grid.x - 1), dim3(512), 0, st, a);
   } else {
     if (KEYS == 128 || pos == 0)
       hipLaunchKernelGGL((context_attention_kernel<D, KEYS, SUB, IdxT, int64_t, false, GEN>), grid, dim3(kThreads), 0,
@@ -1150,8 +1152,9 @@ int group_shift_of(int32_t group) {
   return s;
 }
 
-int64_t split_bytes(int32_t head_dim) {
-  return kSplitGroups * (8 * (head_dim > 64 ? partial_floats<128>() : partial_floats<64>()) + sizeof(Cut));
+// Workspace of 2^shift workgroups.
+int64_t split_bytes(int32_t head_dim, int shift) {
+  return static_cast<int64_t>(8 * (head_dim > 64 ? partial_floats<128>() : partial_floats<64>()) + sizeof(Cut)) << shift;
 }
 
 }  // namespace
@@ -1192,9 +1195,9 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
   if (out_dtype != AKV_BF16 && out_dtype != AKV_F32)
     return fail(AKV_EINVAL, "akv_context_attention: output must be bf16 or f32");
   if (split && (sliding_window > 0 || n_segments > kMaxSplitSegments || !workspace ||
-                workspace_bytes < split_bytes(head_dim) || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0))
+                workspace_bytes < split_bytes(head_dim, 0) || (reinterpret_cast<uintptr_t>(workspace) & 15) != 0))
     return fail(AKV_EINVAL, "akv_context_attention_split: needs no window, at most %d segments and %lld aligned bytes",
-                kMaxSplitSegments, static_cast<long long>(split_bytes(head_dim)));
+                kMaxSplitSegments, static_cast<long long>(split_bytes(head_dim, 0)));
   if (!q || !k_ext || !v_ext || !out || !qo_indptr || !kv_indptr)
     return fail(AKV_EINVAL, "akv_context_attention: null device pointer");
   // prefix keys are read from the pools through kv_indices
@@ -1262,9 +1265,9 @@ int run_context_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
   if (blocks * kv_heads > 0x7fffffffLL) return fail(AKV_EINVAL, "akv_context_attention: queries too long");
   a.kv_heads = kv_heads;
   a.n_segments = n_segments;
-  a.max_shift = kSplitShift;
+  while (split && a.max_shift < kSplitShift && split_bytes(head_dim, a.max_shift + 1) <= workspace_bytes) ++a.max_shift;
   a.partial = static_cast<float*>(workspace);
-  const dim3 grid = split ? dim3(kSplitGroups)
+  const dim3 grid = split ? dim3(1u << a.max_shift)
                           : dim3(static_cast<unsigned>(blocks * kv_heads), 1u, static_cast<unsigned>(n_segments));
   hipStream_t st = as_stream(stream);
   const bool idx64 = indices_dtype == AKV_I64;
@@ -1371,5 +1374,9 @@ extern "C" int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t
   const double tile = kv_heads > 8 ? 1.06 * 1.08 : 1.06;
   const double split = tile * share * tiles + 5. * (share + 1.) + 9.;
   if (plain <= split) return 0;
-  return split_bytes(head_dim);
+  // no more stretches than the batch can have: a turn of 16 tokens over 1000 keys
+  // takes 9 MB, and 69 MB where all CUs work
+  const SplitShape shape{__builtin_ctz(static_cast<uint32_t>(tokens)), head_dim > 64 ? 6 : 7};
+  const int64_t cost = cost_bound(shape, n_segments, queries, total_prefix);
+  return split_bytes(head_dim, parts_shift(shape, cost, kv_heads, kSplitShift));
 }

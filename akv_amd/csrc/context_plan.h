@@ -82,6 +82,13 @@ AKV_HD int64_t segment_cost(const SplitShape& s, int32_t q, int32_t p) {
          block_cost(s);
 }
 
+// A bound of any head's cost for a batch of these sums.
+AKV_HD int64_t cost_bound(const SplitShape& s, int64_t segments, int64_t queries, int64_t prefix) {
+  const int64_t blocks = (queries >> s.token_shift) + segments;
+  const int64_t tiles = ((queries + prefix) >> s.key_shift) + 2;
+  return blocks * (kFullTile * tiles + block_cost(s));
+}
+
 // log2 of the number of stretches: as many as there are workgroups, unless
 // they would be shorter than kMinStretch.
 AKV_HD int32_t parts_shift(const SplitShape& s, int64_t total, int32_t heads, int32_t max_shift) {

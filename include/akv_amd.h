@@ -452,7 +452,9 @@ int akv_context_attention_sized(const void* q, int64_t q_stride_t,
  * (total_queries and total_prefix: host bounds of the batch's sums), or 0
  * when the plain call is the better one.  The workspace holds nothing between
  * calls; calls that overlap need one each.  At most 64 segments, 16-byte
- * aligned workspace; without one, or with a window, the call is refused.
+ * aligned workspace; without one, or with a window, the call is refused.  A
+ * smaller workspace shares the batch out over fewer workgroups (at the least
+ * one, some 270 KB).
  */
 int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t q_heads,
                                           int32_t kv_heads, int32_t head_dim,

@@ -38,6 +38,12 @@ def test_split_bytes_names_the_batches_it_takes():
     assert need(1, 64, 8, 64, 128, 200, 200, 20000) == 0  # a window
     assert need(65, 64, 8, 64, -1, 6500, 100, 20000) == 0  # too many segments
     assert need(1, 64, 8, 64, -1, 4096, 4096, 20000) == 0  # the plain launch fills the chip
+    # short segments that fill a round of the plain launch
+    assert need(64, 28, 4, 128, -1, 64 * 18, 28, 64 * 1900) == 0
+    assert need(32, 40, 8, 128, -1, 32 * 18, 29, 32 * 2268) == 0
+    # a workspace that goes with the batch
+    assert need(1, 64, 8, 64, -1, 16, 16, 1000) < 10 << 20
+    assert need(1, 64, 8, 64, -1, 200, 200, 20000) > 60 << 20
 
 
 @pytest.mark.parametrize("why,changes", [("window", {27: 128}), ("segments", {15: 65}), ("no workspace", {36: None}),

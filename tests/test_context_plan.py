@@ -155,6 +155,9 @@ int main() {
     }
     const Plan pl = plan_of(b);
     if (!pl.total) continue;
+    int64_t queries = 0, prefix = 0;
+    for (int s = 0; s < n; ++s) queries += b.q[s], prefix += b.p[s];
+    if (pl.total > cost_bound(b.sh, n, queries, prefix)) return std::printf("bound, batch %d\n", id), 1;
     // the closed forms against the sums they stand for
     for (int s = 0; s < n; ++s) {
       int64_t sum = 0;

@@ -112,6 +112,84 @@ def test_split_matches_plain(device, monkeypatch, d, idx, ind, pos, segments):
     assert (got - want).abs().max() <= 2e-2
 
 
+@pytest.mark.parametrize("d,hq,hkv", [(64, 16, 2), (128, 28, 4)])
+@pytest.mark.parametrize("shift", range(9))
+def test_any_workspace(device, monkeypatch, d, hq, hkv, shift):
+    """As many workgroups as the workspace holds parts for, from one up."""
+    q_lens, p_lens = [200, 0, 33], [3000, 10, 1100]
+    whole = 8 * (32768 + 2 * (512 if d == 64 else 256)) + 32  # two parts and a cut, per workgroup
+    workspace = torch.full(((whole << shift) + 64,), 255, dtype=torch.uint8, device=device)
+    monkeypatch.setattr(ca, "_split_workspace", lambda *a: workspace[: whole << shift])
+    c = _case(device, hq, hkv, d, q_lens, p_lens, seed=shift)
+    print(f"split workspace d={d} shift={shift}", flush=True)
+    got, want = _run(device, c, window=-1, positions=False, sinks=None, out_dtype=torch.float32, scale=d ** -0.5)
+    assert np.abs(got - want).max() <= TOL
+    assert (workspace[whole << shift:] == 255).all()
+
+
+def test_without_memory_the_plain_launch_runs(device, monkeypatch):
+    q_lens, p_lens = [40], [3000]
+    assert _split(16, 2, 64, q_lens, p_lens)
+    c = _case(device, 16, 2, 64, q_lens, p_lens, seed=1)
+
+    def run():
+        return _run(device, c, window=-1, positions=False, sinks=None, out_dtype=torch.float32, scale=0.125)
+
+    with monkeypatch.context() as m:
+        m.setattr(ca, "_split_workspace", lambda *a: None)
+        plain, want = run()
+    empty, asked = torch.empty, []
+
+    def no_memory(*args, dtype=None, **kw):
+        if dtype is torch.uint8:
+            asked.append(args)
+            raise torch.OutOfMemoryError("no memory for the workspace")
+        return empty(*args, dtype=dtype, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_memory)
+    got, _ = run()
+    assert len(asked) == 1
+    assert (got == plain).all()
+    assert np.abs(got - want).max() <= TOL
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(64, 64, 8), (128, 32, 8)])
+def test_split_in_a_graph(device, d, hq, hkv):
+    """Replays with other inputs in the same buffers, eager calls between them."""
+    q_lens, p_lens = [70, 9], [2500, 900]
+    assert _split(hq, hkv, d, q_lens, p_lens)
+    nq, slots = sum(q_lens), sum(p_lens) + 8
+    rng = np.random.default_rng(d)
+    g = torch.Generator(device=device).manual_seed(d)
+    q, ke, ve, kp, vp = (torch.empty((n, h, d), dtype=torch.bfloat16, device=device)
+                         for n, h in ((nq, hq), (nq, hkv), (nq, hkv), (slots, hkv), (slots, hkv)))
+    idx = torch.from_numpy((rng.permutation(slots - 1)[: sum(p_lens)] + 1).astype(np.int32)).to(device)
+    qo = torch.tensor([0, 70, 79], dtype=torch.int32, device=device)
+    kv = torch.tensor([0, 2500, 3400], dtype=torch.int32, device=device)
+    out, eager = (torch.zeros((nq, hq, d), dtype=torch.bfloat16, device=device) for _ in range(2))
+
+    def call(o):
+        ca.extend_attention_fwd(q, ke, ve, o, kp, vp, qo, kv, idx, None, True, None, max(q_lens))
+
+    def refill():
+        for t in (q, ke, ve, kp, vp):
+            t.normal_(generator=g)
+
+    refill()
+    call(eager)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(out)
+    for _ in range(4):
+        refill()
+        call(eager)
+        junk = torch.full((80 << 20,), 255, dtype=torch.uint8, device=device)  # where eager workspaces were
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager)
+        del junk
+
+
 # heads, head_dim, queries, prefixes; the last two fill a round of full blocks
 @pytest.mark.parametrize("hq,hkv,d,q_lens,p_lens", [(16, 2, 64, [300, 17], [900, 40]), (32, 1, 64, [65, 9], [700, 20]),
                                                     (128, 1, 64, [7, 33], [600, 530]), (14, 2, 32, [130, 1], [20, 600]),
