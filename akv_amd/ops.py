@@ -15,10 +15,19 @@ from . import _lib
 _KV_DTYPES = {torch.float32: _lib.AKV_F32, torch.float16: _lib.AKV_F16, torch.bfloat16: _lib.AKV_BF16}
 
 
+# without a Stream object around the handle, and without looking whether torch
+# is initialised (the caller's tensors are on a device): together about 1 us of
+# each call.  Private functions, so only where this torch has them.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 def current_stream_handle(device):
-    """hipStream_t of torch's current stream on ``device``, as an int."""
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    return torch._C._cuda_getCurrentRawStream(index)  # no Stream object around the handle
+    """hipStream_t of torch's current stream on ``device`` (a device, its name,
+    its index or None, as for ``torch.cuda.current_stream``), as an int."""
+    if _raw_stream is not None and isinstance(device, torch.device) and device.index is not None:
+        return _raw_stream(device.index)
+    return torch.cuda.current_stream(device).cuda_stream
 
 
 class _on_device:
@@ -31,7 +40,7 @@ class _on_device:
         self.previous = None
 
     def __enter__(self):
-        current = torch._C._cuda_getDevice()  # the caller's tensors are on a device: nothing to initialise
+        current = _raw_device()
         if current != self.index:
             self.previous = current
             torch.cuda.set_device(self.index)
