@@ -7,6 +7,7 @@ error.
 
 import ctypes
 import threading
+import warnings
 from ctypes import c_char_p, c_int32, c_int64, c_void_p
 from pathlib import Path
 
@@ -187,16 +188,19 @@ def load():
 
 def calls():
     """The entry points the wrappers call per step, with native argument
-    conversion (``csrc/native.cpp``); same arguments and results as
-    ``load()``'s functions."""
+    conversion (``csrc/native.cpp``) where it is built for this interpreter;
+    same arguments and results as ``load()``'s functions."""
     global _calls
     if _calls is not None:
         return _calls
     lib = load()
     try:
         from . import _native
-    except ImportError as e:
-        raise RuntimeError("akv_amd native calls not built (_native.so); run `python -m akv_amd.build`") from e
+    except ImportError:
+        warnings.warn("akv_amd's native calls are not built for this Python: ctypes takes 3-4 us more per call "
+                      "(python -m akv_amd.build, with Python's headers)", RuntimeWarning, stacklevel=2)
+        _calls = lib
+        return lib
     with _lock:
         if _calls is None:
             for name in _native.names():

@@ -2,7 +2,9 @@
 
 Every translation unit is compiled to an object under ``akv_amd/_build/``
 in parallel, then linked into one shared library next to this file, beside
-``_native.so``, the extension module through which Python calls it.  Device
+the extension module ``_native`` through which Python calls it (named for the
+interpreter it is built with; without Python's headers it is left out, and the
+wrappers call the library through ctypes).  Device
 code is compiled with ``-ffp-contract=off`` (the Reposition arithmetic must
 round every product and sum separately) and without the packed-fp32
 instructions.
@@ -22,7 +24,7 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 OUT_DIR = HERE / "_build"
 LIBRARY = HERE / "libakv_amd.so"
-NATIVE = HERE / "_native.so"
+NATIVE = HERE / ("_native" + sysconfig.get_config_var("EXT_SUFFIX"))
 ARCH = "gfx950"
 
 HIP_SOURCES = [
@@ -74,10 +76,14 @@ def build(verbose=False):
     tmp = LIBRARY.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", *objects, "-o", str(tmp)])
     os.replace(tmp, LIBRARY)
-    tmp = NATIVE.with_suffix(".so.tmp")
-    _run([hipcc, *COMMON_FLAGS, "-x", "c++", "-shared", "-I" + sysconfig.get_paths()["include"],
-          str(CSRC / "native.cpp"), "-o", str(tmp)])
-    os.replace(tmp, NATIVE)
+    (HERE / "_native.so").unlink(missing_ok=True)  # an earlier build's, which any interpreter would load
+    include = Path(sysconfig.get_paths()["include"])
+    if (include / "Python.h").exists():
+        tmp = NATIVE.with_suffix(".so.tmp")
+        _run([hipcc, *COMMON_FLAGS, "-x", "c++", "-shared", f"-I{include}", str(CSRC / "native.cpp"), "-o", str(tmp)])
+        os.replace(tmp, NATIVE)
+    else:
+        print(f"akv_amd: no Python.h in {include}: the native calls are not built, ctypes stands in")
     return LIBRARY
 
 

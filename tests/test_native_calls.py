@@ -1,11 +1,15 @@
 """The native calls against the ctypes functions they stand for: the same
-results and messages, and ctypes' own errors for arguments of other types."""
+results and messages, and ctypes' own errors for arguments of other types; the
+module is this interpreter's, and ctypes stands in where there is none."""
 
 import ctypes
+import sys
+import sysconfig
 
 import pytest
 
-from akv_amd import _lib
+import akv_amd
+from akv_amd import _lib, build
 
 
 def _zeros(fn):
@@ -37,3 +41,30 @@ def test_other_types_meet_ctypes():
     assert calls.akv_decode_attention_workspace_bytes(True, 1, 64, 1) == lib.akv_decode_attention_workspace_bytes(1, 1, 64, 1)
     assert calls.akv_decode_attention_workspace_bytes(2 ** 32 + 1, 1, 64, 1) == \
         lib.akv_decode_attention_workspace_bytes(2 ** 32 + 1, 1, 64, 1)
+
+
+def test_module_is_named_for_the_interpreter():
+    assert build.NATIVE.name == "_native" + sysconfig.get_config_var("EXT_SUFFIX")
+    assert _lib.calls().__file__ == str(build.NATIVE)
+
+
+def test_ctypes_without_the_module(monkeypatch):
+    monkeypatch.setattr(_lib, "_calls", None)
+    monkeypatch.delattr(akv_amd, "_native", raising=False)
+    monkeypatch.setitem(sys.modules, "akv_amd._native", None)  # as if it could not be imported
+    with pytest.warns(RuntimeWarning, match="native calls are not built"):
+        calls = _lib.calls()
+    assert calls is _lib.load() and _lib.calls() is calls
+    assert calls.akv_decode_attention_workspace_bytes(1, 1, 64, 1) > 0
+
+
+def test_build_without_python_headers(monkeypatch, tmp_path, capsys):
+    """The library is built and the module left out."""
+    ran = []
+    monkeypatch.setattr(build, "_run", lambda cmd: ran.append(cmd) or "")
+    monkeypatch.setattr(build.os, "replace", lambda a, b: None)
+    monkeypatch.setattr(build.sysconfig, "get_paths", lambda: {"include": str(tmp_path)})
+    assert build.build() == build.LIBRARY
+    assert "no Python.h" in capsys.readouterr().out
+    assert not any("native.cpp" in str(a) for cmd in ran for a in cmd)
+    assert any(str(a).endswith("libakv_amd.so.tmp") for cmd in ran for a in cmd)
