@@ -522,16 +522,22 @@ __global__ void __launch_bounds__(256) reposition_generic_kernel(const Repositio
 // stays cheap while the rows of all tokens stay cached.  One sweep then also
 // reads source rows that several requests share (page-16 copy-on-write of a
 // common prefix) while a layer's rows are still cached.  So one sweep when the
-// table rows fit kSweepTableBytes, well inside the 256 MB last-level cache:
+// table rows fit kSweepTableBytes, well inside the 256 MB last-level cache, and
+// a K/V row has kSweepRowBytes; beside shorter rows the table's re-reads weigh
+// more, and its rows must stay in the L2s (kShortRowTableBytes):
 // four Llama-3 requests over a shared 8k prefix, 43k copies and 44 MB of table
 // rows, 1946 us against 2227 in chunks; distinct positions, Llama-3 rows of 16
 // layers, sweep | chunks of 1024: 26 MB 647 | 660 us, 51 MB 1170-1300 | 1310,
 // 102 MB 2411-2707 | 2636, 154 MB 4082 | 3244.  The 32k GPT-OSS request's
 // 12064 copies have 6 MB (chunks of 4096-12288 tokens measured 0.5-1.5%
-// slower).  Above, chunks of kChunkTokens tokens, each swept over every layer
+// slower).  Chunks | sweep by row, 64-dim tables of 20, 45 and 60 MB: 512 B (4
+// bf16 heads x 64, 16 layers) 279 | 265, 630 | 613, 840 | 824 us; 256 B (2 heads,
+// 36 layers) 343 | 352, 770 | 819, 1035 | 1101; 128 B 263 | 281, 606 | 688, 799 |
+// 921; 512 B with a 128-dim table 107 | 105, 243 | 235, 323 | 315.  Above, chunks of kChunkTokens tokens, each swept over every layer
 // before the next (777k Llama-3 copies and 777 MB of table rows: 61% of HBM
 // peak in one sweep, 72 / 75 / 76.7% in chunks of 16384 / 4096 / 1024).
-constexpr int64_t kSweepTableBytes = 64ll << 20;
+constexpr int64_t kSweepTableBytes = 64ll << 20, kShortRowTableBytes = 16ll << 20;
+constexpr int64_t kSweepRowBytes = 512;
 constexpr int64_t kChunkTokens = 1024;
 void geometry(RepositionArgs& a) {
   int tokens = 256 / a.lanes_per_row;
@@ -560,7 +566,9 @@ int launch_typed(RepositionArgs a, int64_t n_tokens, hipStream_t stream, bool ve
     const int64_t blocks = ((n_tokens + a.tokens_per_block - 1) / a.tokens_per_block + 7) / 8 * 8;
     const int64_t groups = (a.n_layers + a.layers_per_block - 1) / a.layers_per_block;
     const int64_t table_bytes = n_tokens * 2 * a.rotary_dim * static_cast<int64_t>(sizeof(CS));
-    const int64_t chunk_tokens = table_bytes <= kSweepTableBytes ? n_tokens : kChunkTokens;
+    const int64_t row_bytes = static_cast<int64_t>(a.n_heads) * a.head_dim * static_cast<int64_t>(sizeof(T));
+    const int64_t sweep_bytes = row_bytes >= kSweepRowBytes ? kSweepTableBytes : kShortRowTableBytes;
+    const int64_t chunk_tokens = table_bytes <= sweep_bytes ? n_tokens : kChunkTokens;
     int64_t chunk = ((chunk_tokens + a.tokens_per_block - 1) / a.tokens_per_block + 7) / 8 * 8;
     if (chunk > blocks) chunk = blocks;
     if (blocks * groups > 0x7fffffffLL)

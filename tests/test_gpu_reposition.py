@@ -193,11 +193,12 @@ def test_chunked_sweep(device, heads, head_dim, layers, moved):
               skip_unmapped=True, same_every=5)
 
 
-@pytest.mark.parametrize("moved", [131072, 131073])
-def test_sweep_or_chunks(device, moved):
+@pytest.mark.parametrize("heads,moved", [(4, 131072), (4, 131073), (1, 32768), (1, 32769)])
+def test_sweep_or_chunks(device, heads, moved):
     """131072 tokens of a 64-dim fp32 table have 64 MiB of cos/sin rows, the
-    most that one sweep takes; one more token goes in 1024-token chunks."""
-    _run_case(device, layers=2, heads=1, head_dim=64, slots=2 * moved + 8, moved=moved, seed=12)
+    most that one sweep takes beside 512-byte K/V rows, and 32768 have 16 MiB,
+    the most beside shorter ones; one more token goes in 1024-token chunks."""
+    _run_case(device, layers=2, heads=heads, head_dim=64, slots=2 * moved + 8, moved=moved, seed=12)
 
 
 def test_skip_unmapped_and_same_position(device):
