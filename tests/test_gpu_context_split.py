@@ -217,3 +217,14 @@ def test_without_the_queries_count(device, monkeypatch, window):
     c = _case(device, 16, 2, 64, [300, 17, 90], [900, 40, 300], seed=window + 2)
     got, want = _run(device, c, window=window, positions=True, sinks=None, out_dtype=torch.bfloat16, scale=0.125)
     assert np.abs(got - want).max() <= TOL
+
+
+@pytest.mark.parametrize("positions", [True, False])
+# the first visible key near the prefix's end, inside it, and at its start
+@pytest.mark.parametrize("window", [1, 128, 500, 3000, 9000, 100000])
+@pytest.mark.parametrize("d", [64, 128])
+def test_windows_over_long_prefixes(device, d, window, positions):
+    """Searches of two and three rounds for the first visible key."""
+    c = _case(device, 8, 1, d, [20, 5, 70], [20000, 4097, 4095], seed=window, slots=24000)
+    got, want = _run(device, c, window=window, positions=positions, sinks=None, out_dtype=torch.float32, scale=d ** -0.5)
+    assert np.abs(got - want).max() <= TOL

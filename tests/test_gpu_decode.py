@@ -165,6 +165,48 @@ def test_indptr_and_last_page(device):
         np.testing.assert_array_equal(last.cpu().numpy(), dec.last_page_lengths(lengths, 16))
 
 
+@pytest.mark.parametrize("batch", [63, 65, 127, 128, 129, 1000, 1023, 1024, 1025])
+def test_indptr_widths(device, batch):
+    """One workgroup as wide as the batch: the edges of its waves and of 1024."""
+    rng = np.random.default_rng(batch)
+    lengths = rng.integers(0, 70000, size=batch)
+    indptr = torch.full((batch + 2,), -9, dtype=torch.int64, device=device)
+    last = torch.full((batch + 1,), -9, dtype=torch.int32, device=device)
+    pt.build_indptr(torch.from_numpy(lengths).to(device), indptr[:-1], last_page_len=last[:-1], page_size=16)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(indptr.cpu().numpy(), np.append(dec.kv_indptr(lengths), -9))
+    np.testing.assert_array_equal(last.cpu().numpy(), np.append(dec.last_page_lengths(lengths, 16), -9))
+
+
+@pytest.mark.parametrize("generated", [0, 3])
+def test_window_lengths_of_long_requests(device, generated):
+    """Searches of one to four rounds (64 probes each) over positions with
+    holes: the first visible key at the start, next to it, inside, at the end
+    and past it, by its own position and by one in the hole before it."""
+    window = 5000
+    rng = np.random.default_rng(generated)
+    rows, seq, want, keep = [], [], [], []
+    for n in (1, 2, 63, 64, 65, 127, 128, 4095, 4096, 4097, 4161, 20000, 262145):
+        pos = np.cumsum(rng.integers(1, 4, size=n)).astype(np.int32) + 9000
+        dev = torch.from_numpy(pos).to(device)
+        keep.append(dev)
+        for first in sorted({0, min(1, n - 1), n // 3, n // 2, n - 1, n}):
+            for lower in ((int(pos[first]), int(pos[first]) - 1) if first < n else (int(pos[-1]) + 1, int(pos[-1]) + 2)):
+                nxt = lower - generated + 1 + window
+                rows.append([dev.data_ptr(), dev.data_ptr(), n, n, nxt, 0])
+                seq.append(n + generated)
+                want.append(int((pos >= lower).sum()) + int((nxt + np.arange(generated) >= lower).sum()))
+    registry = torch.tensor(rows, dtype=torch.int64, device=device)
+    lengths = torch.tensor(seq, dtype=torch.int64, device=device)
+    got = torch.full((len(rows) + 1,), -9, dtype=torch.int32, device=device)
+    starts = torch.empty_like(lengths)
+    print(f"window lengths of {len(rows)} long requests", flush=True)
+    pt.context_window_lengths(registry, torch.arange(len(rows), device=device), lengths, got[:-1], window, starts=starts)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(got.cpu().numpy(), want + [-9])
+    np.testing.assert_array_equal(starts.cpu().numpy(), np.array(seq) - np.array(want))
+
+
 def test_pipeline_compaction_feeds_registry(device):
     """compact_rows outputs serve directly as registry rows (no host round trip)."""
     w = synth.workload("ragged-64")
