@@ -40,6 +40,9 @@ HIP_FLAGS = [
     "-fno-fast-math",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
+# the prefill kernels' tile loops begin on a 32-byte boundary: 4096 tokens over
+# 19441 keys 1340 us without, 1332 with; 2040 over 5000 225.9 and 223.4
+FILE_FLAGS = {"context_attention.hip": ["-falign-loops=32"]}
 
 
 def _hipcc():
@@ -63,7 +66,7 @@ def build(verbose=False):
     jobs = []
     for name in HIP_SOURCES:
         obj = OUT_DIR / (name + ".o")
-        jobs.append([hipcc, *COMMON_FLAGS, *HIP_FLAGS, "-c", str(CSRC / name), "-o", str(obj)])
+        jobs.append([hipcc, *COMMON_FLAGS, *HIP_FLAGS, *FILE_FLAGS.get(name, []), "-c", str(CSRC / name), "-o", str(obj)])
     for name in CXX_SOURCES:
         obj = OUT_DIR / (name + ".o")
         jobs.append([hipcc, *COMMON_FLAGS, "-x", "c++", "-c", str(CSRC / name), "-o", str(obj)])
