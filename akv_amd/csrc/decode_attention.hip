@@ -106,8 +106,8 @@ __device__ __forceinline__ int swz(int r) { return D == 64 ? r & 6 : (r & 7) << 
 // with this pass's rows (12 Llama-3 requests and the like 2-8%).
 //
 // The grid follows the host's bound, so its live workgroups must not depend
-// on where they stand in it: workgroups go round robin to the XCDs, and within
-// an XCD to its shader engines, so a grid whose first chunks are the live (or
+// on where they stand in it: workgroups go round robin to the XCDs and, by what
+// the times show, within an XCD to its shader engines, so a grid whose first chunks are the live (or
 // the long) ones would keep to a few of them.  Its chunks therefore turn from
 // pair to pair, at the period of the XCDs and at 4 and 32 times that, and a
 // request's chunks are equally long.  Without both, and with passes from the
@@ -259,6 +259,9 @@ __global__ void __launch_bounds__(4 * D, 4) decode_attention_partial_kernel(cons
         acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop, acc[t], 0, 0, 0);
       }
     }
+    // this pass's reads are done (lgkmcnt 0) before the next pass's rows are
+    // asked into their place: its slots are here already, so nothing else waits
+    __builtin_amdgcn_s_waitcnt(0xc07f);
     asm volatile("" ::: "memory");
   }
 
