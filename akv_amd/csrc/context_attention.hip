@@ -884,10 +884,10 @@ __global__ void __launch_bounds__(kThreads, SUB == 1 ? 4 : 2) context_attention_
 // The split launch: one workgroup per CU, each with an equal stretch of the
 // batch's cost line (context_plan.h).  It is for batches whose plain grid
 // leaves CUs idle: 200 new tokens over 19441 keys are 32 plain workgroups and
-// took 560 us for the GPT-OSS layer, 95 us here with the merge (the matrix
+// took 560 us for the GPT-OSS layer, 93 us here and 13 in the merge (the matrix
 // cores' share is 52 us; the rest is the cuts, a block's first tile, the parts'
 // 28 MB each way and the second launch); six ragged Llama-3 segments (48-624
-// queries over 4-14k keys) took 594 us, 461 us here.
+// queries over 4-14k keys) took 594 us, 437 us here with the merge.
 //
 // A stretch that starts inside a block leaves that block's part for last: the
 // workgroups of an XCD then all begin at their blocks' first keys and walk
@@ -1338,15 +1338,16 @@ extern "C" int akv_context_attention_split(
 // ones, one round more than they fill), after ~12 us; the
 // split launch shares all tiles out evenly at ~6% more a tile, plus ~10 us for
 // each block a workgroup enters (queries, first tile, result) and ~18 us of
-// its own (the cuts, the second launch).  Measured plain against split, us,
-// GPT-OSS (64 q / 8 KV heads x 64) | Llama-3 (32 / 8 x 128), new tokens over
-// prefix keys: 16 / 1000: 45 / 25 | 39 / 25; 200 / 400: 38 / 42 | 30 / 32;
-// 200 / 1000: 52 / 40 | 46 / 37; 800 / 300: 53 / 56 | 45 / 45; 800 / 5000:
-// 183 / 112 | 185 / 101; 1500 / 5000: 207 / 188 | 207 / 176; 2040 / 19000
-// (one full round): 726 / 780 | 650 / 669; 3000 / 300: 128 / 154 | 109 / 127;
-// 3000 / 5000: 397 / 369 | 388 / 342; 4096 / 19441 (two full rounds): 1310 /
-// 1423 | 1326 / 1381; 6 x 682 / 300: 101 / 113 | 79 / 94; 6 x 682 / 5000: 501
-// / 433 | 502 / 411.
+// its own (the cuts, the second launch).  Measured plain / split, us, GPT-OSS
+// (64 q / 8 KV heads x 64) | Llama-3 (32 / 8 x 128), new tokens over prefix
+// keys: 16 / 1000: 43 / 22 | 38 / 22; 200 / 400: 36 / 37 | 29 / 29; 200 / 1000:
+// 50 / 38 | 46 / 34; 800 / 300: 48 / 47 | 42 / 40; 800 / 5000: 182 / 105 | 184 /
+// 100; 1500 / 5000: 203 / 174 | 204 / 169; 1800 / 5000: 213 / 206 | 215 / 201
+// (the rule says plain); 2040 / 19000 (one full round): 631 / 662 | 642 / 650;
+// 3000 / 300: 117 / 141 | 108 / 120; 3000 / 5000: 385 / 352 | 385 / 340; 4096 /
+// 19441 (two full rounds): 1294 / 1384 | 1321 / 1360; 6 x 682 / 300: 97 / 103 |
+// 77 / 86; 6 x 682 / 1000: 152 / 147 | 138 / 133; 6 x 682 / 5000: 498 / 413 |
+// 499 / 400; 32 x 1 / 2000: 76 / 41 | 76 / 56.
 extern "C" int64_t akv_context_attention_split_bytes(int32_t n_segments, int32_t q_heads, int32_t kv_heads,
                                                      int32_t head_dim, int32_t sliding_window, int64_t total_queries,
                                                      int64_t max_query_len, int64_t total_prefix) {

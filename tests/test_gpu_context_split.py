@@ -113,7 +113,7 @@ def test_split_matches_plain(device, monkeypatch, d, idx, ind, pos, segments):
 
 
 @pytest.mark.parametrize("d,hq,hkv", [(64, 16, 2), (128, 28, 4)])
-@pytest.mark.parametrize("shift", range(9))
+@pytest.mark.parametrize("shift", [0, 1, 2, 5, 8])
 def test_any_workspace(device, monkeypatch, d, hq, hkv, shift):
     """As many workgroups as the workspace holds parts for, from one up."""
     q_lens, p_lens = [200, 0, 33], [3000, 10, 1100]
