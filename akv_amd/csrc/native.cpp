@@ -73,6 +73,7 @@ PyObject* invoke(R (*fn)(A...), PyObject* slow, PyObject* const* args, Py_ssize_
   X(akv_write_extend_rows)                \
   X(akv_decode_attention_workspace_bytes) \
   X(akv_decode_attention)                 \
+  X(akv_context_attention)                \
   X(akv_context_attention_sized)          \
   X(akv_context_attention_split)          \
   X(akv_context_attention_split_bytes)    \
